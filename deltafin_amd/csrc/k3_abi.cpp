@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "k3_internal.h"
+#include "k3_skinny.h"
 
 // Per-position decode layers of one call as one position-batched launch pair
 // (launch_decode_positions) where supported; 0 keeps one layer per position.
@@ -1452,6 +1453,27 @@ int k3_hip_moe_launch(const K3HipGeometryV1* gd, const uint8_t* span, const floa
   if (((uintptr_t)span & 15u) != 0 || ((uintptr_t)gate & 15u) != 0)
     return fail(K3_HIP_E_INVALID, "device MoE: span and gate must be 16-byte aligned");
   hipStream_t st = static_cast<hipStream_t>(stream);
+  // gate, up and the activation in one launch where the shape allows
+  SkinnyOp glu{};
+  glu.kind = SKINNY_FP4;
+  glu.w = span + g.w1p;
+  glu.scales = span + g.w1s;
+  glu.w2 = span + g.w3p;
+  glu.scales2 = span + g.w3s;
+  glu.act = g.act;
+  glu.x = x;
+  glu.x_dtype = K3_DTYPE_F32;
+  glu.y = gate;
+  glu.y_up = up;
+  glu.rows = g.inter;
+  glu.cols = g.hidden;
+  glu.positions = batches;
+  if (skinny_fits(glu)) {
+    const int grc = launch_skinny(glu, KC_GEMV, st);
+    if (grc != K3_HIP_OK) return grc;
+    return launch_gemv(span + g.w2p, span + g.w2s, gate, K3_DTYPE_F32, out, K3_DTYPE_F32, g.hidden,
+                       g.inter, batches, st);
+  }
   int rc = launch_gemv(span + g.w1p, span + g.w1s, x, K3_DTYPE_F32, gate, K3_DTYPE_F32, g.inter,
                        g.hidden, batches, st);
   if (rc == K3_HIP_OK)

@@ -240,7 +240,8 @@ enum { K3_SPINE_KIND_BF16 = 0, K3_SPINE_KIND_INT8 = 1 };
 int spine_fail(int status, const char* fmt, ...);
 // accumulate: y += W x instead of y = W x (one fp32 add per output).
 int spine_gemv(int kind, const void* weights, const float* row_scales, const float* x,
-               float* y, int rows, int cols, int positions, bool accumulate, hipStream_t stream);
+               float* y, int rows, int cols, int positions, bool accumulate, hipStream_t stream,
+               bool any_order = false);
 // One spine projection with the fused forms: w2 (GLU): y = act(W x, W2 x) per
 // row (no accumulate); wb: a second matrix's rows after W's (see below);
 // norm_w: x is first RMS-normed per position,
@@ -264,6 +265,10 @@ struct SpineOp {
   const float* scales_b;
   float* yb;
   int rows_b;
+  // The summation order may depend on the number of positions: several
+  // positions take the matrix cores (k3_skinny.hip) where the shape allows.
+  // Unset, a (row, position) sums in one order whatever the batch.
+  bool any_order;
 };
 int spine_gemv_op(int kind, const SpineOp& op, hipStream_t stream);
 // Matrix-core spine (k3_spine_mfma.hip, BF16 matrices, 1..16 positions, cols a

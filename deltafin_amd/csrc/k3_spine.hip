@@ -24,6 +24,7 @@
 
 #include "k3_device.h"
 #include "k3_launch.h"
+#include "k3_skinny.h"
 
 namespace k3 {
 namespace {
@@ -667,6 +668,27 @@ int spine_gemv_op(int kind, const SpineOp& op, hipStream_t st) {
     return spine_fail(K3_SPINE_E_INVALID, "%s: invalid second matrix", what);
   int rc = preflight(what);
   if (rc != K3_SPINE_OK) return rc;
+  // From two positions (three below 2,048 rows, where the launch is all ramp:
+  // 896 x 7168 at two 9.0 us against 7.8) the matrix cores read each weight
+  // once for all of them; 3584 x 7168 BF16, us at 2 / 4 / 16 / 64 positions:
+  // 14.7 / 22.6 / 68.7 / 241.9 -> 11.0 / 11.2 / 16.7 / 28.0.
+  if (op.any_order && !op.w2 && !op.norm_w && !op.wb && !op.accumulate &&
+      op.positions >= (op.rows < 2048 ? 3 : 2)) {
+    SkinnyOp sk{};
+    sk.kind = kind == K3_SPINE_KIND_BF16 ? SKINNY_BF16 : SKINNY_INT8;
+    sk.w = op.w;
+    sk.row_scales = op.scales;
+    sk.x = op.x;
+    sk.x_dtype = K3_DTYPE_F32;
+    sk.y = op.y;
+    sk.rows = op.rows;
+    sk.cols = op.cols;
+    sk.positions = op.positions;
+    if (skinny_fits(sk)) {
+      if (launch_skinny(sk, KC_SPINE_MFMA, st) == K3_HIP_OK) return K3_SPINE_OK;
+      return spine_fail(K3_SPINE_E_RUNTIME, "%s: %s", what, k3_hip_last_error());
+    }
+  }
   const auto* w = static_cast<const uint8_t*>(op.w);
   const int esize = kind == K3_SPINE_KIND_BF16 ? 2 : 1;
   const uint64_t row_bytes = (uint64_t)op.cols * esize;
@@ -724,7 +746,8 @@ int spine_gemv_op(int kind, const SpineOp& op, hipStream_t st) {
 }
 
 int spine_gemv(int kind, const void* weights, const float* row_scales, const float* x,
-               float* y, int rows, int cols, int positions, bool accumulate, hipStream_t st) {
+               float* y, int rows, int cols, int positions, bool accumulate, hipStream_t st,
+               bool any_order) {
   SpineOp op{};
   op.w = weights;
   op.scales = row_scales;
@@ -734,6 +757,7 @@ int spine_gemv(int kind, const void* weights, const float* row_scales, const flo
   op.cols = cols;
   op.positions = positions;
   op.accumulate = accumulate;
+  op.any_order = any_order;
   return spine_gemv_op(kind, op, st);
 }
 

@@ -1,0 +1,166 @@
+"""Several activation rows against one resident matrix on the matrix cores
+(k3_skinny.hip): the spine projections, MXFP4 GEMVs and the one-expert launch
+at the edges of their tiles, against a float64 reference.
+
+Bound: products are exact in fp32 and every output is a sum of `cols` of them in
+eight partial sums, so a sum passes through at most cols / 8 + 16 roundings of
+2^-24 of the sum of |w x| each (and one of 2^-8 where the output is BF16).
+"""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# rows around 16-row tiles and the row counts where 2 and 4 tiles start
+ROWS = [1, 16, 17, 40, 4100, 8200]
+POSITIONS = [2, 3, 4, 5, 8, 9, 16, 17, 33, 64]
+
+
+def _bound(w, x, cols, ref, bf16_out=False):
+    b = (cols / 8 + 16) * 2.0 ** -24 * (x.abs() @ w.abs().t()) + 1e-30
+    return b + 2.0 ** -8 * ref.abs() if bf16_out else b
+
+
+def _check(out, w, x, cols, tag, bf16_out=False):
+    ref = x @ w.t()
+    err = (out.double() - ref).abs()
+    bad = err > _bound(w, x, cols, ref, bf16_out)
+    assert not bad.any(), f"{tag}: {int(bad.sum())} outputs off, worst {err.max().item():.3e}"
+
+
+def _spine(kind, rows, cols, m, seed):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn(m, cols, generator=g, device="cuda")
+    if kind == "bf16":
+        w = torch.randn(rows, cols, generator=g, device="cuda").to(torch.bfloat16)
+        return w, None, x, w.double()
+    w = torch.randint(-128, 128, (rows, cols), generator=g, device="cuda", dtype=torch.int8)
+    s = torch.rand(rows, generator=g, device="cuda") + 0.5
+    return w, s, x, w.double() * s.double().unsqueeze(1)
+
+
+def _run_spine(kind, w, s, x):
+    from deltafin_amd import spine
+    return spine.bf16_gemv(w, x) if kind == "bf16" else spine.int8_gemv(w, s, x)
+
+
+@pytest.mark.parametrize("kind,cols", [("bf16", 32), ("bf16", 64), ("bf16", 72), ("bf16", 1000),
+                                       ("bf16", 2048), ("int8", 64), ("int8", 144),
+                                       ("int8", 1040), ("int8", 2048)])
+def test_spine_edges(gpu, kind, cols):
+    for i, rows in enumerate(ROWS):
+        for m in POSITIONS if cols in (1000, 1040) else POSITIONS[i % 2::3]:
+            print(f"[gpu-case] {kind} {rows}x{cols} positions {m}", flush=True)
+            w, s, x, w64 = _spine(kind, rows, cols, m, rows + m)
+            _check(_run_spine(kind, w, s, x), w64, x.double(), cols, f"{kind} {rows}x{cols} p{m}")
+
+
+def _mxfp4(rows, cols, seed, lo=117, hi=121):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    p = torch.randint(0, 256, (rows, cols // 2), generator=g, device="cuda", dtype=torch.uint8)
+    s = torch.randint(lo, hi + 1, (rows, cols // 32), generator=g, device="cuda",
+                      dtype=torch.uint8)
+    return p, s
+
+
+def _dequant(p, s):
+    import torch
+    v = [0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0]
+    lut = torch.tensor(v + [-a for a in v], dtype=torch.float64, device="cuda")
+    codes = torch.stack((p & 15, p >> 4), dim=-1).reshape(p.shape[0], -1).long()
+    e = s.double()
+    scale = torch.where(e == 0, 0.0, torch.exp2(e - 127.0))
+    return lut[codes] * scale.repeat_interleave(32, dim=1)
+
+
+@pytest.mark.parametrize("cols", [256, 288, 352, 1056, 2048])
+@pytest.mark.parametrize("x_dtype", ["f32", "bf16"])
+def test_mxfp4_edges(gpu, cols, x_dtype):
+    import torch
+    from deltafin_amd import moe
+    for i, rows in enumerate(ROWS):
+        p, s = _mxfp4(rows, cols, rows)
+        w = _dequant(p, s)
+        # scales at an odd address, which the interface allows
+        odd = torch.empty(s.numel() + 1, dtype=torch.uint8, device="cuda")[1:]
+        odd.copy_(s.reshape(-1))
+        for m in (POSITIONS + [100])[i % 2::2]:
+            print(f"[gpu-case] mxfp4 {rows}x{cols} {x_dtype} rows of x {m}", flush=True)
+            x = torch.randn(m, cols, device="cuda").to(
+                torch.float32 if x_dtype == "f32" else torch.bfloat16)
+            for out in (torch.float32, torch.bfloat16):
+                y = moe.mxfp4_gemv(p, odd, x, rows, cols, out_dtype=out)
+                _check(y, w, x.double(), cols, f"mxfp4 {rows}x{cols} {x_dtype} m{m}",
+                       out == torch.bfloat16)
+
+
+@pytest.mark.parametrize("hidden,inter", [(256, 256), (3584, 3072), (1056, 352), (224, 64)])
+def test_expert_rows(gpu, hidden, inter):
+    """moe_launch at 1..17 rows (224 / 64: below a whole line, the separate launches)."""
+    import torch
+    from deltafin_amd import moe
+    g = moe.geometry(hidden, inter, moe.K3_ACT_SITU)
+    off = moe.span_offsets(g)
+    span = torch.empty(off["span"], dtype=torch.uint8, device="cuda").random_(0, 256)
+    mats = {}
+    for name, a, b, c, r, k in (("gate", "w1p", "w1s", "w2p", inter, hidden),
+                                ("down", "w2p", "w2s", "w3p", hidden, inter),
+                                ("up", "w3p", "w3s", "span", inter, hidden)):
+        span[off[b]:off[c]].random_(117, 122)
+        mats[name] = _dequant(span[off[a]:off[b]].reshape(r, -1), span[off[b]:off[c]].reshape(r, -1))
+    for m in (1, 2, 4, 7, 8, 16, 17):
+        print(f"[gpu-case] expert {hidden}/{inter} rows {m}", flush=True)
+        x = torch.randn(m, hidden, device="cuda")
+        h, out = moe.moe_launch(g, span, x)
+        gate, up = x.double() @ mats["gate"].t(), x.double() @ mats["up"].t()
+        ref = 4 * torch.tanh(gate / 4) * torch.sigmoid(gate) * (25 * torch.tanh(up / 25))
+        # the activation's slopes are at most 1.1 |up| and 4: the sums' bounds scaled by
+        # them, and a few roundings of its own
+        tol = (4.0 + 1.1 * up.abs()) * (_bound(mats["gate"], x.double(), hidden, gate)
+                                        + _bound(mats["up"], x.double(), hidden, up)) \
+            + 2.0 ** -20 * (ref.abs() + 1e-3)
+        assert ((h.double() - ref).abs() <= tol).all(), f"h {hidden}/{inter} m{m}"
+        _check(out, mats["down"], h.double(), inter, f"expert {hidden}/{inter} m{m}")
+
+
+def test_non_finite_inputs(gpu):
+    """Infinities and NaN give what plain fp32 sums give: an infinite activation
+    or weight its signed infinity, a NaN scale byte a NaN row, and a scale that
+    overflows BF16 codes the finite result of its small products."""
+    import torch
+    from deltafin_amd import moe
+    inf = float("inf")
+    for kind in ("bf16", "int8"):
+        w, s, x, w64 = _spine(kind, 40, 1040, 5, 3)
+        x[1, 17] = inf
+        x[2, 900] = -inf
+        x[3, 5] = float("nan")
+        # finite, where rounding it to BF16 would not be (int8: below the row scale's reach)
+        x[4, 33] = 3.4028e38 if kind == "bf16" else 1e36
+        if kind == "bf16":
+            w[7, 100] = inf
+            w64 = w.double()
+        y = _run_spine(kind, w, s, x)
+        ref = torch.stack([(x[i].double() * w64).sum(1) for i in range(5)])
+        ref = torch.where(ref.abs() > 3.4028235e38, torch.sign(ref) * inf, ref)
+        assert torch.equal(torch.isnan(y), torch.isnan(ref)), kind
+        assert torch.equal(torch.isinf(y), torch.isinf(ref)), kind
+        assert torch.equal(y[torch.isinf(y)].double(), ref[torch.isinf(ref)]), kind
+        fin = torch.isfinite(ref)
+        assert ((y.double() - ref)[fin].abs() <= 1e-4 * ref[fin].abs() + 1e-2).all(), kind
+    p, s = _mxfp4(40, 512, 5)
+    s[3, 7] = 255   # NaN row
+    s[4, :] = 0     # zero row
+    s[5, 2] = 254   # 2^127: codes above 2 overflow BF16
+    p[5, 32:48] = 0x77  # all codes 6.0
+    for dt in (torch.float32, torch.bfloat16):
+        x = torch.randn(6, 512, device="cuda").to(dt)
+        x[:, 64:96] = x[:, 64:96] * 2.0 ** -130
+        w = _dequant(p, s)
+        y = moe.mxfp4_gemv(p, s, x, 40, 512).double()
+        assert torch.isnan(y[:, 3]).all() and not torch.isnan(y[:, [0, 1, 2, 4, 5, 6]]).any()
+        assert (y[:, 4] == 0).all()
+        ref = x.double() @ w.t()
+        keep = [i for i in range(40) if i != 3]
+        assert ((y - ref)[:, keep].abs() <= 1e-4 * (x.double().abs() @ w[keep].abs().t())).all()
