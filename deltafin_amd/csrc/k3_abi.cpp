@@ -869,10 +869,8 @@ int verify_table(const Geo& g, const EdgeTable& tbl, const void* x, int x_dtype,
 }
 
 // ---------------------------------------------------------------- MoE block
-// Positions from which the block's BF16 spine runs on the matrix cores.
-#ifndef K3_SPINE_MFMA_MIN_POSITIONS
-#define K3_SPINE_MFMA_MIN_POSITIONS 3
-#endif
+// Positions from which the block's spine projections run on the matrix cores.
+constexpr int kBlockSkinnyPositions = 3;
 static_assert(sizeof(K3HipMoeSpineV1) == 144, "K3HipMoeSpineV1 layout changed");
 
 // Block workspace: the expert workspace, then logits [P, E], routed_in and
@@ -886,8 +884,6 @@ struct BlockBufs {
   float* routed_out;
   float* gate;
   float* up;
-  uint8_t* terms;   // BF16 activation terms of the matrix-core spine (P >= 3)
-  uint8_t* terms2;  // the hidden rows' terms for the side stream's shared gate/up
 };
 
 uint64_t block_layout(const K3HipMoeSpineV1& sp, const Geo& g, int max_positions,
@@ -909,12 +905,6 @@ uint64_t block_layout(const K3HipMoeSpineV1& sp, const Geo& g, int max_positions
   take(b ? &b->routed_out : nullptr, P * sp.routed_hidden);
   take(b ? &b->gate : nullptr, P * sp.shared_intermediate);
   take(b ? &b->up : nullptr, P * sp.shared_intermediate);
-  const int wmax = (int)std::max(sp.hidden, std::max(sp.routed_hidden, sp.shared_intermediate));
-  if (b) b->terms = base + off;
-  off += align256(spine_mfma_terms_bytes(max_positions, wmax));
-  if (b) b->terms2 = base + off;  // the side stream's: hidden rows, then the shared h
-  off += align256(spine_mfma_terms_bytes(
-      max_positions, (int)std::max(sp.hidden, sp.shared_intermediate)));
   return off;
 }
 
@@ -1051,77 +1041,16 @@ int k3_hip_moe_block_device(const K3HipMoeSpineV1* spine, const K3HipGeometryV1*
   // after the fork joins first, so the caller's stream is never ahead of the
   // side work.
   SideWork side(st);
-  // 3..16 positions of a BF16 spine: every projection on the matrix cores
-  // from BF16 activation terms (the fp32 kernels are bound by LDS and FMAs
-  // there); the steps and their order are the same.
-  const bool matrices_aligned =
-      ((reinterpret_cast<uintptr_t>(sp.router) | reinterpret_cast<uintptr_t>(sp.routed_down) |
-        reinterpret_cast<uintptr_t>(sp.routed_up) | reinterpret_cast<uintptr_t>(sp.shared_gate) |
-        reinterpret_cast<uintptr_t>(sp.shared_up) | reinterpret_cast<uintptr_t>(sp.shared_down)) &
-       15u) == 0;
-  if (P >= K3_SPINE_MFMA_MIN_POSITIONS && kind == K3_SPINE_KIND_BF16 && matrices_aligned &&
-      spine_mfma_supported(kind, P, R, H) && spine_mfma_supported(kind, P, S, H) &&
-      spine_mfma_supported(kind, P, H, R) && spine_mfma_supported(kind, P, H, S)) {
-    auto mm = [&](const void* w, const uint8_t* terms, float* y, int rows, int cols, bool acc,
-                  hipStream_t s, const char* step) {
-      return from_spine(spine_mfma_gemv(w, terms, y, rows, cols, P, acc, s), step);
-    };
-    auto split = [&](const float* x, int cols, uint8_t* terms, hipStream_t s) {
-      return from_spine(spine_mfma_split(x, P, cols, terms, s), "term split");
-    };
-    // shared gate and up from the hidden rows' terms (already split into
-    // `terms` when `split_first` is false), then h = situ(gate, up)
-    auto shared_glu = [&](uint8_t* terms, bool split_first, hipStream_t s) -> int {
-      int r;
-      if ((split_first && (r = split(hidden, H, terms, s))) ||
-          (r = mm(sp.shared_gate, terms, b.gate, S, H, false, s, "shared_gate")) ||
-          (r = mm(sp.shared_up, terms, b.up, S, H, false, s, "shared_up")))
-        return r;
-      return launch_activation(b.gate, b.up, b.gate, (int64_t)P * S, K3_ACT_SITU, s);
-    };
-    // With the side stream the shared expert reads its own copy of the hidden
-    // rows' terms (the main stream's buffer is reused for the routed output
-    // while the side work may still run), and the side stream also splits
-    // its h into that buffer for shared_down, off the main stream's path.
-    if (side.parallel() && (rc = side.fork([&](hipStream_t s) {
-                              const int r = shared_glu(b.terms2, true, s);
-                              return r ? r : split(b.gate, S, b.terms2, s);
-                            })))
-      return rc;
-    // The router logits stay on the fp32 kernels at every P: each position's
-    // logit is then summed in the same order whatever the batch (the fp32
-    // spine kernels reduce every (row, position) identically), so a hidden row
-    // routes to the same experts in a 1-token decode and in a verify batch.
-    if ((rc = from_spine(spine_gemv(kind, sp.router, sp.router_scales, hidden, b.logits, E, H, P,
-                                    false, st), "router")) ||
-        (rc = split(hidden, H, b.terms, st)) ||
-        (rc = mm(sp.routed_down, b.terms, b.routed_in, R, H, false, st, "routed_down")) ||
-        (!side.parallel() && (rc = shared_glu(b.terms, false, st))))
-      return rc;
-    if ((rc = launch_route_sigmoid_bias(b.logits, sp.router_bias, E, top_k, P, ws.ids, ws.w,
-                                        route_ids, route_weights, st)))
-      return rc;
-    if ((rc = experts_on_device_routes(g, bank, expert_stride, E, P, top_k, b.routed_in,
-                                       b.routed_out, ws, st)))
-      return rc;
-    // the routed RMS norm writes routed_up's terms in the same launch
-    rc = spine_rms_norm_terms(b.routed_out, sp.routed_norm, b.routed_out, P, R, K3_RMS_EPSILON,
-                              b.terms, st);
-    if (rc == K3_SPINE_E_UNSUPPORTED) {
-      if ((rc = from_spine(spine_rms_norm(b.routed_out, sp.routed_norm, b.routed_out, P, R,
-                                          K3_RMS_EPSILON, st), "routed RMS norm")) ||
-          (rc = split(b.routed_out, R, b.terms, st)))
-        return rc;
-    } else if ((rc = from_spine(rc, "routed RMS norm"))) {
-      return rc;
-    }
-    if ((rc = mm(sp.routed_up, b.terms, out, H, R, false, st, "routed_up")) ||
-        (rc = side.join()))
-      return rc;
-    if (!side.parallel() && (rc = split(b.gate, S, b.terms, st))) return rc;
-    return mm(sp.shared_down, side.parallel() ? b.terms2 : b.terms, out, H, S, true, st,
-              "shared_down");
-  }
+  // From three positions every projection but the router runs on the matrix
+  // cores (k3_skinny.hip) where its shape allows.  The router logits stay on
+  // the fp32 kernels at every P: each position's logit is then summed in the
+  // same order whatever the batch, so a hidden row routes to the same experts
+  // in a 1-token decode and in a verify batch.
+  const bool skinny = P >= kBlockSkinnyPositions;
+  auto project = [&](const void* w, const float* scales, const float* x, float* y, int rows,
+                     int cols, bool acc, const char* step) {
+    return from_spine(spine_gemv(kind, w, scales, x, y, rows, cols, P, acc, st, skinny), step);
+  };
   // the shared expert: h = situ(gate, up), one launch reading each gate row
   // and its up row together (two launches and the activation where the shape
   // has no fused form); h overwrites gate
@@ -1137,6 +1066,7 @@ int k3_hip_moe_block_device(const K3HipMoeSpineV1* spine, const K3HipGeometryV1*
     glu.rows = S;
     glu.cols = H;
     glu.positions = P;
+    glu.any_order = skinny;
     int r = spine_gemv_op(kind, glu, s);
     if (r == K3_SPINE_E_UNSUPPORTED) {
       if ((r = from_spine(spine_gemv(kind, sp.shared_gate, sp.shared_gate_scales, hidden, b.gate,
@@ -1152,29 +1082,29 @@ int k3_hip_moe_block_device(const K3HipMoeSpineV1* spine, const K3HipGeometryV1*
   if (side.parallel() && (rc = side.fork(shared_glu))) return rc;
   // prepare: router logits and routed_down (one launch over both matrices,
   // which read the same hidden rows, where the shape allows), then the route
-  SpineOp pre{};
-  pre.w = sp.router;
-  pre.scales = sp.router_scales;
-  pre.x = hidden;
-  pre.y = b.logits;
-  pre.rows = E;
-  pre.cols = H;
-  pre.positions = P;
-  pre.wb = sp.routed_down;
-  pre.scales_b = sp.routed_down_scales;
-  pre.yb = b.routed_in;
-  pre.rows_b = R;
-  rc = spine_gemv_op(kind, pre, st);
-  if (rc == K3_SPINE_E_UNSUPPORTED) {
-    if ((rc = from_spine(spine_gemv(kind, sp.router, sp.router_scales, hidden, b.logits, E, H, P,
-                                    false, st), "router")))
-      return rc;
-    if ((rc = from_spine(spine_gemv(kind, sp.routed_down, sp.routed_down_scales, hidden,
-                                    b.routed_in, R, H, P, false, st), "routed_down")))
-      return rc;
-  } else if ((rc = from_spine(rc, "router + routed_down"))) {
-    return rc;
+  rc = K3_SPINE_E_UNSUPPORTED;
+  if (!skinny) {
+    SpineOp pre{};
+    pre.w = sp.router;
+    pre.scales = sp.router_scales;
+    pre.x = hidden;
+    pre.y = b.logits;
+    pre.rows = E;
+    pre.cols = H;
+    pre.positions = P;
+    pre.wb = sp.routed_down;
+    pre.scales_b = sp.routed_down_scales;
+    pre.yb = b.routed_in;
+    pre.rows_b = R;
+    rc = spine_gemv_op(kind, pre, st);
+    if (rc != K3_SPINE_E_UNSUPPORTED && (rc = from_spine(rc, "router + routed_down"))) return rc;
   }
+  if (rc == K3_SPINE_E_UNSUPPORTED &&
+      ((rc = from_spine(spine_gemv(kind, sp.router, sp.router_scales, hidden, b.logits, E, H, P,
+                                   false, st), "router")) ||
+       (rc = project(sp.routed_down, sp.routed_down_scales, hidden, b.routed_in, R, H, false,
+                     "routed_down"))))
+    return rc;
   if ((rc = launch_route_sigmoid_bias(b.logits, sp.router_bias, E, top_k, P, ws.ids, ws.w,
                                       route_ids, route_weights, st)))
     return rc;
@@ -1185,30 +1115,29 @@ int k3_hip_moe_block_device(const K3HipMoeSpineV1* spine, const K3HipGeometryV1*
   if (!side.parallel() && (rc = shared_glu(st))) return rc;
   // complete: routed_up over the routed RMS norm (staged normalised by the
   // projection itself where the shape allows), + shared_down h (one fp32 add)
-  SpineOp up{};
-  up.w = sp.routed_up;
-  up.scales = sp.routed_up_scales;
-  up.x = b.routed_out;
-  up.y = out;
-  up.rows = H;
-  up.cols = R;
-  up.positions = P;
-  up.norm_w = sp.routed_norm;
-  up.eps = K3_RMS_EPSILON;
-  rc = spine_gemv_op(kind, up, st);
-  if (rc == K3_SPINE_E_UNSUPPORTED) {
-    if ((rc = from_spine(spine_rms_norm(b.routed_out, sp.routed_norm, b.routed_out, P, R,
-                                        K3_RMS_EPSILON, st), "routed RMS norm")))
-      return rc;
-    if ((rc = from_spine(spine_gemv(kind, sp.routed_up, sp.routed_up_scales, b.routed_out, out,
-                                    H, R, P, false, st), "routed_up")))
-      return rc;
-  } else if ((rc = from_spine(rc, "routed_up"))) {
-    return rc;
+  rc = K3_SPINE_E_UNSUPPORTED;
+  if (!skinny) {
+    SpineOp up{};
+    up.w = sp.routed_up;
+    up.scales = sp.routed_up_scales;
+    up.x = b.routed_out;
+    up.y = out;
+    up.rows = H;
+    up.cols = R;
+    up.positions = P;
+    up.norm_w = sp.routed_norm;
+    up.eps = K3_RMS_EPSILON;
+    rc = spine_gemv_op(kind, up, st);
+    if (rc != K3_SPINE_E_UNSUPPORTED && (rc = from_spine(rc, "routed_up"))) return rc;
   }
+  if (rc == K3_SPINE_E_UNSUPPORTED &&
+      ((rc = from_spine(spine_rms_norm(b.routed_out, sp.routed_norm, b.routed_out, P, R,
+                                       K3_RMS_EPSILON, st), "routed RMS norm")) ||
+       (rc = project(sp.routed_up, sp.routed_up_scales, b.routed_out, out, H, R, false,
+                     "routed_up"))))
+    return rc;
   if ((rc = side.join())) return rc;  // h from the side stream
-  return from_spine(spine_gemv(kind, sp.shared_down, sp.shared_down_scales, b.gate, out, H, S, P,
-                               true, st), "shared_down");
+  return project(sp.shared_down, sp.shared_down_scales, b.gate, out, H, S, true, "shared_down");
 }
 
 uint64_t k3_hip_geometry_span(uint32_t hidden, uint32_t intermediate) {

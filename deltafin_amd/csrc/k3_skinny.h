@@ -14,13 +14,15 @@ struct SkinnyOp {
   const void* w;               // [rows, cols], row-major
   const uint8_t* scales;       // SKINNY_FP4: E8M0 [rows, cols / 32]
   const float* row_scales;     // SKINNY_INT8: [rows]
-  const void* w2;              // SKINNY_FP4: a second matrix (GLU), y = act(w . x, w2 . x)
+  const float* row_scales2;
+  const void* w2;              // a second matrix (GLU): y = act(w . x, w2 . x)
   const uint8_t* scales2;
   int act;                     // GLU: K3_ACT_*
   const void* x;               // [positions, cols]
   int x_dtype;                 // K3_DTYPE_*; BF16 only for SKINNY_FP4 without w2
   void* y;                     // [positions, rows]
   float* y_up;                 // GLU: w2 . x when non-null
+  const float* add;            // y += add [positions, rows] (fp32, no GLU; may be y)
   int out_bf16;
   int rows, cols, positions;
 };

@@ -57,10 +57,11 @@ constexpr int operands() {
 struct SkinnyArgs {
   const uint8_t* w[2];   // weights; [1] = up with kGlu
   const uint8_t* sc[2];  // MXFP4 scale planes
-  const float* rs;       // int8 row scales
+  const float* rs[2];    // int8 row scales
   const void* x;
   void* y;
-  float* y_up;  // kGlu: receives up . x when non-null
+  float* y_up;       // kGlu: receives up . x when non-null
+  const float* add;  // added to an fp32 result when non-null
   int rows, cols, P;
   int lines;      // 128-byte lines of a row, the last one possibly partial
   int tail;       // bytes of the last line
@@ -490,7 +491,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_skinny(const SkinnyArgs args
         if (w < S) sum += pk[w * TLT * NB * 256];
       if (!(fabsf(sum) < INFINITY))
         sum = plain_dot<kW, XT>(args.w[k], args.sc[k], args.x, row, p0 + p, args.cols);
-      if constexpr (kW == SKINNY_INT8) sum *= args.rs[row];
+      if constexpr (kW == SKINNY_INT8) sum *= args.rs[k][row];
       v[k] = sum;
     }
     const uint64_t yi = (uint64_t)(p0 + p) * rows + row;
@@ -502,6 +503,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_skinny(const SkinnyArgs args
     if (args.out_bf16) {
       static_cast<uint16_t*>(args.y)[yi] = f32_to_bf16_bits(out);
     } else {
+      if (!kGlu && args.add) out = args.add[yi] + out;
       static_cast<float*>(args.y)[yi] = out;
     }
   }
@@ -548,11 +550,20 @@ bool go_rows(int TL, const SkinnyArgs& a, hipStream_t st, TimedLaunch& tl) {
   return go_tiles<kW, XT, 4>(TL, a, st, tl);
 }
 
+// Tiles of gate and as many of up: two of each where one would leave more
+// workgroups than CUs (MXFP4, with its longer lines, always one).
+template <int kW, int RQ>
+bool go_glu_tiles(int TL, const SkinnyArgs& a, hipStream_t st, TimedLaunch& tl) {
+  if constexpr (kW != SKINNY_FP4)
+    if (TL > 1) return go<kW, float, RQ, 2, true, 2>(a, st, tl);
+  return go<kW, float, RQ, 1, true, depth<kW, 2>()>(a, st, tl);
+}
+
 template <int kW>
-bool go_glu(const SkinnyArgs& a, hipStream_t st, TimedLaunch& tl) {
-  if (a.P <= 4) return go<kW, float, 1, 1, true, 1>(a, st, tl);
-  if (a.P <= 8) return go<kW, float, 2, 1, true, 1>(a, st, tl);
-  return go<kW, float, 4, 1, true, 1>(a, st, tl);
+bool go_glu(int TL, const SkinnyArgs& a, hipStream_t st, TimedLaunch& tl) {
+  if (a.P <= 4) return go_glu_tiles<kW, 1>(TL, a, st, tl);
+  if (a.P <= 8) return go_glu_tiles<kW, 2>(TL, a, st, tl);
+  return go_glu_tiles<kW, 4>(TL, a, st, tl);
 }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
@@ -568,7 +579,7 @@ bool skinny_fits(const SkinnyOp& op) {
          row_bytes >= (op.kind == SKINNY_FP4 ? 128u : 64u) && op.cols <= 65536 &&
          op.positions <= (1 << 19) && (uint64_t)op.positions * op.cols <= (1u << 28) &&
          (uint64_t)op.positions * op.rows <= INT32_MAX && aligned16(op.w) && aligned16(op.x) &&
-         (!op.w2 || (aligned16(op.w2) && op.kind == SKINNY_FP4 && op.x_dtype == K3_DTYPE_F32));
+         (!op.w2 || (aligned16(op.w2) && op.x_dtype == K3_DTYPE_F32));
 }
 
 int launch_skinny(const SkinnyOp& op, int kernel_class, hipStream_t st) {
@@ -577,7 +588,9 @@ int launch_skinny(const SkinnyOp& op, int kernel_class, hipStream_t st) {
   a.w[1] = static_cast<const uint8_t*>(op.w2);
   a.sc[0] = op.scales;
   a.sc[1] = op.scales2;
-  a.rs = op.row_scales;
+  a.rs[0] = op.row_scales;
+  a.rs[1] = op.row_scales2;
+  a.add = op.add;
   a.x = op.x;
   a.y = op.y;
   a.y_up = op.y_up;
@@ -606,14 +619,13 @@ int launch_skinny(const SkinnyOp& op, int kernel_class, hipStream_t st) {
   while (TL < 4 && (int64_t)((a.rows + 16 * TL - 1) / (16 * TL)) * pb > cus) TL *= 2;
   TimedLaunch tl(kernel_class, st);
   bool ok;
-  if (op.w2)
-    ok = go_glu<SKINNY_FP4>(a, st, tl);
-  else if (op.kind == SKINNY_BF16)
-    ok = go_rows<SKINNY_BF16, float>(TL, a, st, tl);
+  const bool glu = op.w2 != nullptr;
+  if (op.kind == SKINNY_BF16)
+    ok = glu ? go_glu<SKINNY_BF16>(TL, a, st, tl) : go_rows<SKINNY_BF16, float>(TL, a, st, tl);
   else if (op.kind == SKINNY_INT8)
-    ok = go_rows<SKINNY_INT8, float>(TL, a, st, tl);
+    ok = glu ? go_glu<SKINNY_INT8>(TL, a, st, tl) : go_rows<SKINNY_INT8, float>(TL, a, st, tl);
   else if (op.x_dtype == K3_DTYPE_F32)
-    ok = go_rows<SKINNY_FP4, float>(TL, a, st, tl);
+    ok = glu ? go_glu<SKINNY_FP4>(TL, a, st, tl) : go_rows<SKINNY_FP4, float>(TL, a, st, tl);
   else
     ok = go_rows<SKINNY_FP4, uint16_t>(TL, a, st, tl);
   if (!ok) {
