@@ -35,6 +35,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "k3_device.h"
 #include "k3_internal.h"
@@ -45,6 +46,8 @@ namespace k3 {
 
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(1))) const u32x2 gu32x2;
 
 // ======================================================================
 // split activation rows into fp8 terms (k3_terms.h)
@@ -65,18 +68,17 @@ __global__ __launch_bounds__(256) void k_split_terms(const SrcT* __restrict__ sr
 // Workgroup b takes units b, b + NWG, ... and each wave walks the flattened
 // (unit, K-step pair) items: weights two items ahead, activation terms one.
 //
-// Parity split.  An MFMA row needs its four lanes (l % 16 equal) to hold the
-// same weight row, and a load instruction streams fastest when it covers
-// whole 128-byte lines.  Each weight row p of a tile of 8 therefore takes two
-// MFMA rows, 2p + h, h = 0 for the even K step of the pair and 1 for the odd
-// one: lane l (i = l % 16, g = l / 16) loads row i / 2, K step ks + i % 2,
-// block g, and one dwordx4 load of a tile covers 8 rows x one full 128-byte
-// line (K steps ks, ks + 1).  Two MFMAs per tile and item use that same A
-// register, one with the activation terms of step ks (valid in the even
-// rows of its result) and one with those of step ks + 1 (valid in the odd
-// rows); lane (q, n) then sums rows 4q + 0 / 4q + 1 and 4q + 2 / 4q + 3 of
-// the two accumulators into weight rows 2q and 2q + 1 of the tile for token
-// n.  The other rows are never read.
+// Tile pairs.  An MFMA row needs its four lanes (l % 16 equal) to hold the same
+// weight row, and a load instruction streams fastest when it covers whole
+// 128-byte lines: lane l (i = l % 16, g = l / 16) loads row i / 2 of a tile of 8
+// rows, K step ks + i % 2, block g, one dwordx4 load per tile and line (K steps
+// ks, ks + 1).  Neighbouring lanes of two tiles exchange halves (one DPP step), so
+// that one register holds K step ks of 16 rows and the other K step ks + 1: MFMA
+// row 2 i is row i of the first tile, 2 i + 1 row i of the second.  The unit's
+// scaled products are what bounds fp32 x and the down rows, with three terms:
+// multiplying each tile's two K steps in separate MFMA rows instead, which
+// needs no exchange and twice the MFMAs, ran the K3 block's 16-position
+// gate/up at 462 us against 416 (5.7 -> 6.3 TB/s) and down at 235 against 209.
 //
 // At a unit's last item every wave writes its tiles' partial sums to LDS
 // (two slots by unit parity, one barrier per unit) and wave w sums tile w
@@ -84,14 +86,14 @@ __global__ __launch_bounds__(256) void k_split_terms(const SrcT* __restrict__ sr
 // and stores its tokens' rows.
 //
 // Every address is in range by construction: units are below U * n_rb,
-// rows below the matrix's rows, K steps below K / 128, and lanes whose token
-// column is empty read token 0's activation row (their columns are never
-// stored).
+// rows below the matrix's rows, K steps below K / 128, and packed rows past an
+// expert's last repeat it (the columns past its tokens are never stored).
 struct MfmaPlan {
   const uint8_t* uptr[K3_HIP_MAX_EDGES];
   int uoff[K3_HIP_MAX_EDGES + 1];
   int brow[K3_HIP_MAX_EDGES];  // activation row of the i-th grouped edge
   int orow[K3_HIP_MAX_EDGES];  // output row (the edge) of the i-th grouped edge
+  int over[4];                 // per wave: an expert with more than 2 (bit 0), 4 (bit 1) quads
 };
 
 // Scale block of a wave's unit: its rows' E8M0 bytes for its K steps, KS
@@ -100,12 +102,30 @@ struct MfmaPlan {
 // lane) and parked in the wave's LDS region as [tile][row][K step].
 constexpr int kScaleLoads = 16;
 
+// Packed activation terms: at most kPackQuads quads of (token, term) rows, 256
+// bytes of two K steps and 8 scale bytes each.
+constexpr int kPackQuads = 4;
+constexpr int kPackBytes = 4 * kPackQuads * 256 + 64 * 8;  // every lane stores 8 bytes
+
 template <int kTiles>
 struct MfmaA {  // weights: streamed from HBM, two items in flight
   u32x4 a[kTiles];
 };
+// Activation terms of K steps ks, ks + 1 (one item ahead), in one of two forms.
+// Packed (NQ > 0): the expert's rows (token, term) as 256 contiguous bytes each,
+// four rows per load, and their scale bytes in one more load, redistributed
+// through LDS; NQ quads hold every row of the batch's experts.  Direct (NQ = 0):
+// every lane loads its own operand runs, 4 T + T loads per item however few
+// tokens there are.  Loads that hit the L2 cost the weight stream nearly as much
+// as the weights do (a streaming probe at 7.1 TB/s falls to 6.4 with one such
+// load per weight load and to 5.4 with two).
+template <int T, int NQ>
+struct MfmaB {
+  u32x4 r[NQ];
+  u32x2 s;
+};
 template <int T>
-struct MfmaB {  // activation terms of K steps ks, ks + 1: L2-resident, one item ahead
+struct MfmaB<T, 0> {
   u32x4 b[T][2][2];  // [term][K step][K runs 16 g.. and 64 + 16 g..]
   uint32_t sb[T][2];
 };
@@ -120,21 +140,34 @@ __device__ __forceinline__ v8i b_operand(u32x4 lo, u32x4 hi) {
   return r;
 }
 
+// a[0], a[1] (8 rows x two K steps each, lane parity the K step) -> K step 0 and
+// K step 1 of 16 rows.
+__device__ __forceinline__ void pair_halves(u32x4 (&a)[2], bool odd) {
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const uint32_t send = odd ? a[0][d] : a[1][d];
+    const uint32_t recv =
+        (uint32_t)__builtin_amdgcn_update_dpp(0, (int)send, 0xB1, 0xf, 0xf, false);  // lane ^ 1
+    a[0][d] = odd ? recv : a[0][d];
+    a[1][d] = odd ? a[1][d] : recv;
+  }
+}
+
 // Activation terms are re-read by every unit of their expert: ordinary
 // (cached) loads, unlike the streamed weight chunks.
 __device__ __forceinline__ u32x4 load_b16(const uint8_t* p) { return *(gu32x4*)(p); }
 
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(1))) const u32x2 gu32x2;
 
 template <bool kGlu, int NT, int T>
 __global__ __launch_bounds__(256, 2) void k_verify_mfma(const Geo g, const Workspace ws,
                                                         const uint8_t* __restrict__ bq,
                                                         const uint8_t* __restrict__ bqs,
-                                                        int n_brows, float* __restrict__ out) {
+                                                        int n_brows, int max_edges,
+                                                        float* __restrict__ out) {
   constexpr int kM = kGlu ? 2 : 1;
   constexpr int kTiles = kM * NT;
-  extern __shared__ float2 red[];  // [2][S][kTiles][64] sums, then [S][64 * kScaleLoads] scales
+  // [2][S][kTiles][64] sums, then [S][64 * kScaleLoads] scales, then [S] packed rows
+  extern __shared__ __attribute__((aligned(16))) float2 red[];
   __shared__ MfmaPlan pl;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -150,16 +183,46 @@ __global__ __launch_bounds__(256, 2) void k_verify_mfma(const Geo g, const Works
   const uint64_t wp[2] = {kGlu ? g.w1p : g.w2p, g.w3p};
   const uint64_t wsc[2] = {kGlu ? g.w1s : g.w2s, g.w3s};
 
-  const int U = min(ws.plan->n_unique, K3_HIP_MAX_EDGES);
-  const int n_edges = min(ws.plan->n_edges, K3_HIP_MAX_EDGES);
-  for (int i = threadIdx.x; i < U; i += blockDim.x) pl.uptr[i] = ws.uptr[i];
-  for (int i = threadIdx.x; i <= U; i += blockDim.x) pl.uoff[i] = min(max(ws.uoff[i], 0), n_edges);
-  for (int i = threadIdx.x; i < n_edges; i += blockDim.x) {
-    const int e = min(max(ws.uedges[i], 0), n_edges - 1);
-    pl.orow[i] = e;
-    pl.brow[i] = min(max(kGlu ? ws.epos[e] : e, 0), n_brows - 1);
+  // The plan into LDS: every array's loads in flight at once (max_edges bounds
+  // them; only the edges' positions depend on another load), then the most
+  // tokens of any expert, which chooses how the terms are loaded (below).
+  constexpr int kPer = K3_HIP_MAX_EDGES / 64;  // entries per thread of the smallest workgroup
+  const uint8_t* up[kPer];
+  int uo[kPer], ue[kPer];
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const int i = (int)threadIdx.x + r * (int)blockDim.x;
+    if (i < max_edges) {
+      up[r] = ws.uptr[i];
+      uo[r] = ws.uoff[i];
+      ue[r] = ws.uedges[i];
+    }
   }
+  const int U = min(ws.plan->n_unique, max_edges);
+  const int n_edges = min(ws.plan->n_edges, max_edges);
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const int i = (int)threadIdx.x + r * (int)blockDim.x;
+    if (i < U) {
+      pl.uptr[i] = up[r];
+      pl.uoff[i] = min(max(uo[r], 0), n_edges);
+    }
+    if (i < n_edges) {
+      const int e = min(max(ue[r], 0), n_edges - 1);
+      pl.orow[i] = e;
+      pl.brow[i] = min(max(kGlu ? ws.epos[e] : e, 0), n_brows - 1);
+    }
+  }
+  if (threadIdx.x == 0) pl.uoff[U] = n_edges;
   __syncthreads();
+  int most = 0;
+  for (int i = threadIdx.x; i < U; i += blockDim.x) most = max(most, pl.uoff[i + 1] - pl.uoff[i]);
+  const bool w2 = __any(most * T > 8), w4 = __any(most * T > 16);
+  if (lane == 0) pl.over[wave] = (w2 ? 1 : 0) | (w4 ? 2 : 0);
+  __syncthreads();
+  int over = 0;
+  for (int w = 0; w < S; ++w) over |= pl.over[w];
+  const bool over2 = (over & 1) != 0, over4 = (over & 2) != 0;
   const int n_units = U * n_rb;
   const int NWG = gridDim.x;
   const int b0 = blockIdx.x;
@@ -168,42 +231,10 @@ __global__ __launch_bounds__(256, 2) void k_verify_mfma(const Geo g, const Works
   const int n_items = iters * KP;
 
   typedef MfmaA<kTiles> ItemA;
-  typedef MfmaB<T> ItemB;
   // Loads address a wave-uniform base (scalar registers: the expert's span,
   // the activation terms) plus a 32-bit per-lane offset, so each load needs
   // one VGPR of address instead of two.
   const uint32_t a_lane = (uint32_t)(prow * rowb) + 64u * par + 16u * qb;  // + row block, tile, K
-  auto load_b = [&](ItemB& it, int i) {
-    const int ui = i / KP;
-    const int unit = b0 + ui * NWG;
-    const int ks = wave * KS + 2 * (i - ui * KP);
-    const int uid = unit / n_rb;
-    const int e0 = pl.uoff[uid], m = pl.uoff[uid + 1] - e0;
-    const bool tok = r16 < m;
-    const int brow = pl.brow[min(e0 + (tok ? r16 : 0), n_edges - 1)];
-    const uint32_t boff = (uint32_t)(brow * T * K) + 128u * ks + 16u * qb;
-    const uint32_t bsoff = (uint32_t)(brow * T * (int)srowb) + 4u * ks;
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-      if (tok) {
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          it.b[t][k][0] = load_b16(bq + (boff + (uint32_t)(t * K + 128 * k)));
-          it.b[t][k][1] = load_b16(bq + (boff + (uint32_t)(t * K + 128 * k) + 64u));
-        }
-        const u32x2 sv = *(gu32x2*)(bqs + (bsoff + (uint32_t)(t * (int)srowb)));
-        it.sb[t][0] = sv.x;
-        it.sb[t][1] = sv.y;
-      } else {
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          it.b[t][k][0] = u32x4{0u, 0u, 0u, 0u};
-          it.b[t][k][1] = u32x4{0u, 0u, 0u, 0u};
-          it.sb[t][k] = 0u;
-        }
-      }
-    }
-  };
   // Scale block addressing: dword j*64 + lane of the block is tile
   // idx / (8 KS), row (idx / KS) % 8, K step idx % KS of the wave's range.
   const int n_sdw = kTiles * 8 * KS;  // <= 64 * kScaleLoads (host check)
@@ -298,69 +329,197 @@ __global__ __launch_bounds__(256, 2) void k_verify_mfma(const Geo g, const Works
   const uint32_t sh = 8u * qb;  // this lane group's byte in each scale dword
   uint32_t* sblk_lds = reinterpret_cast<uint32_t*>(red + (size_t)2 * S * kTiles * 64) +
                        (size_t)wave * 64 * kScaleLoads;
-  auto compute = [&](const ItemA& ia, const ItemB& ib, int i) {
-    const int ui = i / KP;
-    const int kp = i - ui * KP;
-    if (kp == 0) {
+  // This wave's packed term rows: [4 kPackQuads rows][16] pieces of 16 bytes (piece
+  // c of row r at c ^ r % 16, which spreads the row-wise stores and the token-wise
+  // reads over the banks), then the rows' scale bytes.
+  u32x4* rows_lds = reinterpret_cast<u32x4*>(
+      reinterpret_cast<uint8_t*>(red) + (size_t)2 * S * kTiles * 64 * sizeof(float2) +
+      (size_t)S * 64 * kScaleLoads * sizeof(uint32_t) + (size_t)wave * kPackBytes);
+  u32x2* rows_sc = reinterpret_cast<u32x2*>(rows_lds + 64 * kPackQuads);
+
+  auto body = [&](auto quads) {
+    constexpr int NQ = decltype(quads)::value;
+    typedef MfmaB<T, NQ> ItemB;
+    uint32_t boff[NQ > 0 ? NQ : 1], bsoff = 0;  // packed: row offsets of the terms' unit
+    auto load_b = [&](ItemB& it, int i) {
+      const int ui = i / KP;
+      const int unit = b0 + ui * NWG;
+      const int ks = wave * KS + 2 * (i - ui * KP);
+      const int uid = unit / n_rb;
+      const int e0 = pl.uoff[uid], m = pl.uoff[uid + 1] - e0;
+      if constexpr (NQ > 0) {
+        if (i == ui * KP) {
+          auto row_at = [&](int row) {  // rows past the expert's last repeat it
+            const int r = min(row, m * T - 1);
+            const int tok = r / T;
+            return pl.brow[min(e0 + tok, n_edges - 1)] * T + (r - tok * T);
+          };
 #pragma unroll
-      for (int t = 0; t < kTiles; ++t) acc[t] = make_float2(0.0f, 0.0f);
+          for (int n = 0; n < NQ; ++n)
+            boff[n] = __umul24((uint32_t)row_at(4 * n + qb), (uint32_t)K) + 16u * r16;  // see load_s
+          bsoff = __umul24((uint32_t)row_at(min(lane, 4 * NQ - 1)), (uint32_t)srowb);
+        }
 #pragma unroll
-      for (int j = 0; j < kScaleLoads; ++j)
-        if (64 * j < n_sdw) sblk_lds[64 * j + lane] = sblk[j];
-    }
-    // the A scale of this lane: its weight row, K step 2 kp + par, block qb
-    const uint32_t* sa_row = sblk_lds + prow * KS + 2 * kp + par;
-    // Per tile: the item's two K steps' products, each over all terms, then the
-    // valid rows folded into the tile's accumulator (rows 4 qb + 0 and + 2 of
-    // the even step's result, + 1 and + 3 of the odd step's).
+        for (int n = 0; n < NQ; ++n) it.r[n] = load_b16(bq + (boff[n] + 128u * ks));
+        it.s = *(gu32x2*)(bqs + (bsoff + 4u * ks));
+      } else {
+        const bool tok = r16 < m;
+        const int brow = pl.brow[min(e0 + (tok ? r16 : 0), n_edges - 1)];
+        const uint32_t o = (uint32_t)(brow * T * K) + 128u * ks + 16u * qb;
+        const uint32_t so = (uint32_t)(brow * T * (int)srowb) + 4u * ks;
 #pragma unroll
-    for (int t = 0; t < kTiles; ++t) {
-      const int sa = (int)((sa_row[t * 8 * KS] >> sh) & 0xffu);
-      v4f d[2];
+        for (int t = 0; t < T; ++t) {
+          if (tok) {
 #pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        d[k] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int k = 0; k < 2; ++k) {
+              it.b[t][k][0] = load_b16(bq + (o + (uint32_t)(t * K + 128 * k)));
+              it.b[t][k][1] = load_b16(bq + (o + (uint32_t)(t * K + 128 * k) + 64u));
+            }
+            const u32x2 sv = *(gu32x2*)(bqs + (so + (uint32_t)(t * (int)srowb)));
+            it.sb[t][0] = sv.x;
+            it.sb[t][1] = sv.y;
+          } else {
 #pragma unroll
-        for (int j = 0; j < T; ++j) {
-          const int sb = (int)((ib.sb[j][k] >> sh) & 0xffu);
-          d[k] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-              a_operand(ia.a[t]), b_operand(ib.b[j][k][0], ib.b[j][k][1]), d[k],
-              4 /* A: fp4 */, 0 /* B: fp8 e4m3 */, 0, sa, 0, sb);
+            for (int k = 0; k < 2; ++k) {
+              it.b[t][k][0] = u32x4{0u, 0u, 0u, 0u};
+              it.b[t][k][1] = u32x4{0u, 0u, 0u, 0u};
+              it.sb[t][k] = 0u;
+            }
+          }
         }
       }
-      acc[t].x += d[0][0] + d[1][1];
-      acc[t].y += d[0][2] + d[1][3];
-    }
-    if (kp == KP - 1) epilogue(ui);
-  };
+    };
+    auto compute = [&](const ItemA& ia, const ItemB& ib, int i) {
+      const int ui = i / KP;
+      const int kp = i - ui * KP;
+      if constexpr (NQ > 0) {  // a wave's LDS operations run in order: no barrier
+#pragma unroll
+        for (int n = 0; n < NQ; ++n) {
+          const int row = 4 * n + qb;
+          rows_lds[16 * row + (r16 ^ (row & 15))] = ib.r[n];
+        }
+        rows_sc[lane] = ib.s;  // unconditional: under a branch its load would sink to here
+        __builtin_amdgcn_wave_barrier();
+      }
+      if (kp == 0) {
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) acc[t] = make_float2(0.0f, 0.0f);
+#pragma unroll
+        for (int j = 0; j < kScaleLoads; ++j)
+          if (64 * j < n_sdw) sblk_lds[64 * j + lane] = sblk[j];
+      }
+      // Tiles in pairs: neighbouring lanes exchange halves so that a[0] holds K
+      // step ks of 16 rows and a[1] K step ks + 1 (MFMA row 2 i the first tile's
+      // row i, row 2 i + 1 the second's); per pair the two K steps' products, each
+      // over all terms, then folded into the tiles' accumulators.  The A scale of
+      // this lane: its weight row, that K step, block qb.
+      const uint32_t* sa_row = sblk_lds + (par * 8 + prow) * KS + 2 * kp;
+      constexpr int kPairs = kTiles / 2;
+      constexpr int kStep = NQ > 0 ? 2 : 1;  // pairs per pass over the terms
+#pragma unroll
+      for (int q0 = 0; q0 < kPairs; q0 += kStep) {
+        v4f d[2][kStep];
+        u32x4 a[kStep][2];
+        int sa[kStep][2];
+#pragma unroll
+        for (int q = 0; q < kStep; ++q) {
+          a[q][0] = ia.a[2 * (q0 + q)];
+          a[q][1] = ia.a[2 * (q0 + q) + 1];
+          pair_halves(a[q], par != 0);
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            sa[q][k] = (int)((sa_row[(q0 + q) * 16 * KS + k] >> sh) & 0xffu);
+            d[k][q] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+#pragma unroll
+          for (int j = 0; j < T; ++j) {
+            v8i bo;
+            int sb;
+            if constexpr (NQ > 0) {
+              // lanes past the expert's tokens read some row of the region (their
+              // columns are never stored)
+              const int row = min(r16 * T + j, 4 * NQ - 1);
+              const u32x4* rp = rows_lds + 16 * row;
+              bo = b_operand(rp[(8 * k + qb) ^ (row & 15)], rp[(8 * k + 4 + qb) ^ (row & 15)]);
+              sb = (int)((reinterpret_cast<const uint32_t*>(rows_sc + row)[k] >> sh) & 0xffu);
+            } else {
+              bo = b_operand(ib.b[j][k][0], ib.b[j][k][1]);
+              sb = (int)((ib.sb[j][k] >> sh) & 0xffu);
+            }
+#pragma unroll
+            for (int q = 0; q < kStep; ++q)
+              d[k][q] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                  a_operand(a[q][k]), bo, d[k][q], 4 /* A: fp4 */, 0 /* B: fp8 e4m3 */, 0, sa[q][k],
+                  0, sb);
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < kStep; ++q) {
+          float2& lo = acc[2 * (q0 + q)];
+          float2& hi = acc[2 * (q0 + q) + 1];
+          lo.x += d[0][q][0] + d[1][q][0];
+          hi.x += d[0][q][1] + d[1][q][1];
+          lo.y += d[0][q][2] + d[1][q][2];
+          hi.y += d[0][q][3] + d[1][q][3];
+        }
+        if constexpr (NQ > 0) __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (NQ > 0) __builtin_amdgcn_wave_barrier();
+      if (kp == KP - 1) epilogue(ui);
+    };
 
-  // Issue order per item (every path issues the same loads after the terms,
-  // so the compiler's wait counts stay exact): the scale block of item i + 3
-  // when it starts a unit, the activation terms of item i + 1, the weights
-  // of item i + 2 (past the end: the last item again).  Waiting for item
-  // i + 1's terms then leaves item i + 2's weights in flight, so the weight
-  // stream stays two items deep while the terms need one buffer.
-  ItemA A0, A1;
-  ItemB Bc;
-  auto maybe_load_s = [&](int i) {
-    if (i < n_items && i - (i / KP) * KP == 0) load_s(i);
-  };
-  load_s(0);
-  load_b(Bc, 0);
-  load_a(A0, 0);
-  load_a(A1, min(1, n_items - 1));
-  for (int i = 0;; i += 2) {
+    // Issue order per item (every path issues the same loads after the terms,
+    // so the compiler's wait counts stay exact): the scale block of item i + 3
+    // when it starts a unit, the activation terms of item i + 1, the weights
+    // of item i + 2 (past the end: the last item again).  Waiting for item
+    // i + 1's terms then leaves item i + 2's weights in flight, so the weight
+    // stream stays two items deep while the terms need one buffer.
+    ItemA A0, A1;
+    ItemB Bc;
+    auto maybe_load_s = [&](int i) {
+      if (i < n_items && i - (i / KP) * KP == 0) load_s(i);
+    };
+    load_s(0);
+    load_b(Bc, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    load_a(A0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    load_a(A1, min(1, n_items - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    // No exits or conditions on the products inside the loop, and every load in
+    // it used on every path: otherwise the paths past a load merge into the wait
+    // counts at the loop's head, or the load sinks to where it is used.  With an
+    // odd n_items the last product is one item past the end: it multiplies the
+    // last item's loads into a sum that no epilogue reads (units are at least
+    // three items long).
+    int i = 0;
+    for (; i + 2 < n_items; i += 2) {
+      compute(A0, Bc, i);
+      maybe_load_s(i + 3);
+      load_b(Bc, i + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      load_a(A0, i + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(A1, Bc, i + 1);
+      maybe_load_s(i + 4);
+      load_b(Bc, i + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      load_a(A1, min(i + 3, n_items - 1));
+      __builtin_amdgcn_sched_barrier(0);
+    }
     compute(A0, Bc, i);
-    if (i + 1 >= n_items) break;
-    maybe_load_s(i + 3);
-    load_b(Bc, i + 1);
-    load_a(A0, min(i + 2, n_items - 1));
+    load_b(Bc, min(i + 1, n_items - 1));
     compute(A1, Bc, i + 1);
-    if (i + 2 >= n_items) break;
-    maybe_load_s(i + 4);
-    load_b(Bc, i + 2);
-    load_a(A1, min(i + 3, n_items - 1));
-  }
+  };
+  if (!over2)
+    body(std::integral_constant<int, 2>{});
+  else if (!over4)
+    body(std::integral_constant<int, kPackQuads>{});
+  else
+    body(std::integral_constant<int, 0>{});
 }
 
 // ======================================================================
@@ -373,7 +532,7 @@ namespace {
 // takes hidden sizes that are multiples of 128, so these units always fit).
 // Each keeps two items of weights and one of
 // activation terms within the 256 VGPRs of two waves per SIMD without
-// spilling (fp32 x at 4 tiles: 253, down at 8: 246).  More weight bytes per
+// spilling (fp32 x at 4 tiles: 238, down at 8: 237).  More weight bytes per
 // item measured faster: fp32 x at 2 tiles (16 rows each) ran the K3 block's
 // 16-position gate/up at 607-634 µs against 465 µs at 4, and down at 7 tiles
 // the preset-2 16-position verify's down at 288-289 µs against 266 at 8.
@@ -430,16 +589,19 @@ int mfma_launch(const Geo& g, int n_edges, const Workspace& ws, const uint8_t* b
                           kGlu ? K3_MFMA_GLU_WAVES : K3_MFMA_DOWN_WAVES);
   if (S < 1) return fail(K3_HIP_E_INVALID, "verify: no column split fits this geometry");
   const int max_units = n_edges * (rows / (8 * NT));
-  // eight resident waves per CU (two per SIMD, the kernel's register budget)
-  const int grid = std::max(1, std::min((8 / S) * std::max(1, device_cu_count()), max_units));
   const unsigned lds = (unsigned)(2 * S * kTiles * 64 * sizeof(float2) +
-                                  (size_t)S * 64 * kScaleLoads * sizeof(uint32_t));
+                                  (size_t)S * 64 * kScaleLoads * sizeof(uint32_t) +
+                                  (size_t)S * kPackBytes);
+  // eight resident waves per CU (two per SIMD, the kernel's register budget),
+  // or what a CU's 160 KB of LDS hold (one-wave workgroups)
+  const int per_cu = std::min(8 / S, (int)(160 * 1024 / (lds + sizeof(MfmaPlan))));
+  const int grid = std::max(1, std::min(per_cu * std::max(1, device_cu_count()), max_units));
   const void* kfn = reinterpret_cast<const void*>(k_verify_mfma<kGlu, NT, T>);
   if (!lds_fits(kfn, 64 * S, lds))
     return fail(K3_HIP_E_EXEC, "verify: %u B of LDS per workgroup not available", lds);
   TimedLaunch tl(kGlu ? KC_GLU_MFMA : KC_DOWN_MFMA, st);
   launch_timed(tl, k_verify_mfma<kGlu, NT, T>, dim3(grid), dim3(64 * S), lds, st, g, ws, bq, bqs,
-               n_brows, out);
+               n_brows, n_edges, out);
   return launched(tl, kGlu ? "verify gate/up (mfma) launch" : "verify down (mfma) launch");
 }
 

@@ -322,3 +322,36 @@ def test_verify_mfma_spans_above_2g_low_word(gpu, verify_mode):
                                         g.hidden, g.intermediate, g.activation, x[p])
         assert oracle.cond_rel_err(out[p], ref, mag, g.intermediate) <= TOL, f"position {p}"
     del buf
+
+
+@pytest.mark.parametrize("xdt", ["bf16", "f32"])
+@pytest.mark.parametrize("preset_id", [1, 2])
+def test_verify_mfma_tokens_per_expert(gpu, verify_mode, preset_id, xdt):
+    """One to sixteen tokens per expert: the batch's largest count chooses how
+    the activation terms are loaded (two row quads, four, or lane by lane), and
+    with two or three terms per token the counts 2, 4, 5 and 8 are the last of
+    each.  A position's sums do not depend on the other positions, so every
+    batch repeats the largest one's outputs bit for bit."""
+    import torch
+    from deltafin_amd import moe
+    g = moe.preset(preset_id)
+    verify_mode(_lib.VERIFY_UNION_MFMA)
+    spans = [oracle.synth_expert(57, e, g.hidden, g.intermediate) for e in range(3)]
+    d = [_t(sp) for sp in spans]
+    x = np.random.default_rng(5).standard_normal((16, g.hidden)).astype(np.float32)
+    x = _bf16_round(x) if xdt == "bf16" else x
+    w = np.array([0.5, 0.3, 0.2], np.float32)
+    outs = {}
+    for m in (16, 1, 2, 3, 4, 5, 6, 8, 9):
+        say(f"verify mfma tokens per expert preset={preset_id} x={xdt} m={m}")
+        xd = (_bf16(x[:m]) if xdt == "bf16" else _t(x[:m])).reshape(m, g.hidden)
+        ws = moe.workspace(g, 3 * m, m)
+        out = moe.moe_verify(g, d * m, w.tolist() * m, list(range(0, 3 * m + 1, 3)), xd, ws)
+        torch.cuda.synchronize()
+        outs[m] = out.cpu().numpy()
+        assert np.array_equal(outs[m], outs[16][:m]), f"m={m}"
+    for p in (0, 15):
+        ref, mag = oracle.moe_layer_f64(spans, w.astype(np.float64), g.hidden, g.intermediate,
+                                        g.activation, x[p])
+        err = oracle.cond_rel_err(outs[16][p], ref, mag, g.intermediate)
+        assert err <= TOL, f"position {p}: {err:.3e}"
