@@ -874,8 +874,8 @@ constexpr int kBlockSkinnyPositions = 3;
 static_assert(sizeof(K3HipMoeSpineV1) == 144, "K3HipMoeSpineV1 layout changed");
 
 // Block workspace: the expert workspace, then logits [P, E], routed_in and
-// routed_out [P, R], shared gate and up [P, S] (h overwrites gate), each
-// 256-byte aligned.
+// routed_out [P, R], shared gate and up [P, S] (h overwrites gate), the shared
+// expert's output [P, H], each 256-byte aligned.
 struct BlockBufs {
   uint8_t* expert_ws;
   uint64_t expert_ws_bytes;
@@ -884,6 +884,7 @@ struct BlockBufs {
   float* routed_out;
   float* gate;
   float* up;
+  float* shared;
 };
 
 uint64_t block_layout(const K3HipMoeSpineV1& sp, const Geo& g, int max_positions,
@@ -905,6 +906,7 @@ uint64_t block_layout(const K3HipMoeSpineV1& sp, const Geo& g, int max_positions
   take(b ? &b->routed_out : nullptr, P * sp.routed_hidden);
   take(b ? &b->gate : nullptr, P * sp.shared_intermediate);
   take(b ? &b->up : nullptr, P * sp.shared_intermediate);
+  take(b ? &b->shared : nullptr, P * sp.hidden);
   return off;
 }
 
@@ -1032,12 +1034,12 @@ int k3_hip_moe_block_device(const K3HipMoeSpineV1* spine, const K3HipGeometryV1*
   const int P = n_positions, H = (int)sp.hidden, R = (int)sp.routed_hidden;
   const int S = (int)sp.shared_intermediate, E = (int)sp.experts;
   int rc;
-  // The shared expert's gate/up needs only the hidden rows, so it runs on the
-  // side stream where there is one, beside the router, the routed experts and
-  // routed_up (the two streams' kernels share the CUs and fill each other's
-  // ramps), and the caller's stream waits for it only before shared_down.
-  // The next call's fork is recorded after this call's shared_down, so the
-  // side stream never overwrites h that is still to be read.  Every return
+  // The shared expert needs only the hidden rows, so all of it runs on the side
+  // stream where there is one, beside the router and the routed experts (the
+  // two streams' kernels share the CUs and fill each other's ramps), and the
+  // caller's stream waits for its output only before routed_up, which adds it.
+  // The next call's fork is recorded after this call's routed_up, so the side
+  // stream never overwrites an output that is still to be read.  Every return
   // after the fork joins first, so the caller's stream is never ahead of the
   // side work.
   SideWork side(st);
@@ -1048,10 +1050,10 @@ int k3_hip_moe_block_device(const K3HipMoeSpineV1* spine, const K3HipGeometryV1*
   // in a 1-token decode and in a verify batch.
   const bool skinny = P >= kBlockSkinnyPositions;
   auto project = [&](const void* w, const float* scales, const float* x, float* y, int rows,
-                     int cols, bool acc, const char* step) {
-    return from_spine(spine_gemv(kind, w, scales, x, y, rows, cols, P, acc, st, skinny), step);
+                     int cols, const float* add, hipStream_t s, const char* step) {
+    return from_spine(spine_gemv(kind, w, scales, x, y, rows, cols, P, add, s, skinny), step);
   };
-  // the shared expert: h = situ(gate, up), one launch reading each gate row
+  // the shared expert's h = situ(gate, up), one launch reading each gate row
   // and its up row together (two launches and the activation where the shape
   // has no fused form); h overwrites gate
   auto shared_glu = [&](hipStream_t s) -> int {
@@ -1070,16 +1072,21 @@ int k3_hip_moe_block_device(const K3HipMoeSpineV1* spine, const K3HipGeometryV1*
     int r = spine_gemv_op(kind, glu, s);
     if (r == K3_SPINE_E_UNSUPPORTED) {
       if ((r = from_spine(spine_gemv(kind, sp.shared_gate, sp.shared_gate_scales, hidden, b.gate,
-                                     S, H, P, false, s), "shared_gate")))
+                                     S, H, P, nullptr, s), "shared_gate")))
         return r;
       if ((r = from_spine(spine_gemv(kind, sp.shared_up, sp.shared_up_scales, hidden, b.up, S,
-                                     H, P, false, s), "shared_up")))
+                                     H, P, nullptr, s), "shared_up")))
         return r;
       return launch_activation(b.gate, b.up, b.gate, (int64_t)P * S, K3_ACT_SITU, s);
     }
     return from_spine(r, "shared gate/up");
   };
-  if (side.parallel() && (rc = side.fork(shared_glu))) return rc;
+  auto shared_expert = [&](hipStream_t s) -> int {
+    const int r = shared_glu(s);
+    return r ? r : project(sp.shared_down, sp.shared_down_scales, b.gate, b.shared, H, S, nullptr, s,
+                           "shared_down");
+  };
+  if (side.parallel() && (rc = side.fork(shared_expert))) return rc;
   // prepare: router logits and routed_down (one launch over both matrices,
   // which read the same hidden rows, where the shape allows), then the route
   rc = K3_SPINE_E_UNSUPPORTED;
@@ -1101,8 +1108,8 @@ int k3_hip_moe_block_device(const K3HipMoeSpineV1* spine, const K3HipGeometryV1*
   }
   if (rc == K3_SPINE_E_UNSUPPORTED &&
       ((rc = from_spine(spine_gemv(kind, sp.router, sp.router_scales, hidden, b.logits, E, H, P,
-                                   false, st), "router")) ||
-       (rc = project(sp.routed_down, sp.routed_down_scales, hidden, b.routed_in, R, H, false,
+                                   nullptr, st), "router")) ||
+       (rc = project(sp.routed_down, sp.routed_down_scales, hidden, b.routed_in, R, H, nullptr, st,
                      "routed_down"))))
     return rc;
   if ((rc = launch_route_sigmoid_bias(b.logits, sp.router_bias, E, top_k, P, ws.ids, ws.w,
@@ -1112,9 +1119,10 @@ int k3_hip_moe_block_device(const K3HipMoeSpineV1* spine, const K3HipGeometryV1*
   if ((rc = experts_on_device_routes(g, bank, expert_stride, E, P, top_k, b.routed_in,
                                      b.routed_out, ws, st)))
     return rc;
-  if (!side.parallel() && (rc = shared_glu(st))) return rc;
+  if (!side.parallel() && (rc = shared_expert(st))) return rc;
+  if ((rc = side.join())) return rc;  // the shared expert's output
   // complete: routed_up over the routed RMS norm (staged normalised by the
-  // projection itself where the shape allows), + shared_down h (one fp32 add)
+  // projection itself where the shape allows), + the shared expert (one fp32 add)
   rc = K3_SPINE_E_UNSUPPORTED;
   if (!skinny) {
     SpineOp up{};
@@ -1125,6 +1133,7 @@ int k3_hip_moe_block_device(const K3HipMoeSpineV1* spine, const K3HipGeometryV1*
     up.rows = H;
     up.cols = R;
     up.positions = P;
+    up.add = b.shared;
     up.norm_w = sp.routed_norm;
     up.eps = K3_RMS_EPSILON;
     rc = spine_gemv_op(kind, up, st);
@@ -1133,11 +1142,10 @@ int k3_hip_moe_block_device(const K3HipMoeSpineV1* spine, const K3HipGeometryV1*
   if (rc == K3_SPINE_E_UNSUPPORTED &&
       ((rc = from_spine(spine_rms_norm(b.routed_out, sp.routed_norm, b.routed_out, P, R,
                                        K3_RMS_EPSILON, st), "routed RMS norm")) ||
-       (rc = project(sp.routed_up, sp.routed_up_scales, b.routed_out, out, H, R, false,
+       (rc = project(sp.routed_up, sp.routed_up_scales, b.routed_out, out, H, R, b.shared, st,
                      "routed_up"))))
     return rc;
-  if ((rc = side.join())) return rc;  // h from the side stream
-  return project(sp.shared_down, sp.shared_down_scales, b.gate, out, H, S, true, "shared_down");
+  return K3_HIP_OK;
 }
 
 uint64_t k3_hip_geometry_span(uint32_t hidden, uint32_t intermediate) {

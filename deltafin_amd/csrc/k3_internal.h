@@ -238,12 +238,13 @@ class TimedLaunch {
 // spine surface; failures record their reason through spine_fail.
 enum { K3_SPINE_KIND_BF16 = 0, K3_SPINE_KIND_INT8 = 1 };
 int spine_fail(int status, const char* fmt, ...);
-// accumulate: y += W x instead of y = W x (one fp32 add per output).
+// add (nullable): y = W x + add, [positions, rows], one fp32 add per output.
 int spine_gemv(int kind, const void* weights, const float* row_scales, const float* x,
-               float* y, int rows, int cols, int positions, bool accumulate, hipStream_t stream,
+               float* y, int rows, int cols, int positions, const float* add,
+               hipStream_t stream,
                bool any_order = false);
 // One spine projection with the fused forms: w2 (GLU): y = act(W x, W2 x) per
-// row (no accumulate); wb: a second matrix's rows after W's (see below);
+// row (no add); wb: a second matrix's rows after W's (see below);
 // norm_w: x is first RMS-normed per position,
 // norm_w * (x * rsqrt(mean(x^2) + eps)).  A fused form the shape cannot take
 // returns K3_SPINE_E_UNSUPPORTED before enqueuing anything.
@@ -256,7 +257,7 @@ struct SpineOp {
   const float* x;
   float* y;
   int rows, cols, positions;
-  bool accumulate;
+  const float* add;
   const float* norm_w;
   float eps;
   // A second matrix of the same width over the same x (wb, scales_b: rows_b

@@ -169,7 +169,7 @@ template <int kKind, int NJ, int R, int PG, bool kGlu = false>
 __global__ __launch_bounds__(kSpineThreads, kGlu ? 2 : 4) void k_spine_gemv(
     const uint8_t* __restrict__ w, const float* __restrict__ row_scale,
     const float* __restrict__ x, float* __restrict__ y, int rows, int cols, int positions,
-    int tail_lanes, int accumulate, const uint8_t* __restrict__ w2,
+    int tail_lanes, const float* __restrict__ add, const uint8_t* __restrict__ w2,
     const float* __restrict__ row_scale2, int act, const float* __restrict__ norm_w, float eps) {
   using E = SpineElem<kKind>;
   static_assert(!kGlu || R == 2, "a GLU wave holds one gate row and one up row");
@@ -269,8 +269,8 @@ __global__ __launch_bounds__(kSpineThreads, kGlu ? 2 : 4) void k_spine_gemv(
             float s = wave_sum(acc[r][p]);
             if (kKind == K3_SPINE_KIND_INT8) s *= scale;
             if (lane == 0 && row < rows) {
-              float* yp = y + (uint64_t)(p0 + p) * rows + row;
-              *yp = accumulate ? *yp + s : s;
+              const uint64_t yi = (uint64_t)(p0 + p) * rows + row;
+              y[yi] = add ? add[yi] + s : s;
             }
           }
         }
@@ -289,7 +289,7 @@ template <int kKind, int NJ, int PG>
 __global__ __launch_bounds__(kSpineThreads, 2) void k_spine_stream(
     const uint8_t* __restrict__ w, const float* __restrict__ row_scale,
     const float* __restrict__ x, float* __restrict__ y, int rows, int cols, int positions,
-    int tail_lanes, int accumulate, const float* __restrict__ norm_w, float eps,
+    int tail_lanes, const float* __restrict__ add, const float* __restrict__ norm_w, float eps,
     const uint8_t* __restrict__ wb, const float* __restrict__ row_scale_b, float* __restrict__ yb,
     int rows_a) {
   // Rows [0, rows_a) are w's (output y [P][rows_a]); with wb, rows [rows_a,
@@ -352,7 +352,7 @@ __global__ __launch_bounds__(kSpineThreads, 2) void k_spine_stream(
         if (lane == 0) {
           float* yp = in_a ? y + (uint64_t)p * rows_a + row
                            : yb + (uint64_t)p * rows_b + (row - rows_a);
-          *yp = accumulate ? *yp + s : s;
+          *yp = add ? add[(uint64_t)p * rows_a + row] + s : s;  // add: one matrix only
         }
       }
     }
@@ -381,7 +381,7 @@ template <int kKind>
 __global__ __launch_bounds__(kSpineThreads) void k_spine_gemv_generic(
     const uint8_t* __restrict__ w, const float* __restrict__ row_scale,
     const float* __restrict__ x, float* __restrict__ y, int rows, int cols, int positions,
-    int accumulate) {
+    const float* __restrict__ add) {
   const int lane = threadIdx.x & (kWave - 1);
   const int row = blockIdx.x * kSpineWaves + threadIdx.x / kWave;
   if (row >= rows) return;
@@ -401,8 +401,8 @@ __global__ __launch_bounds__(kSpineThreads) void k_spine_gemv_generic(
     float s = wave_sum(acc);
     if (kKind == K3_SPINE_KIND_INT8) s *= row_scale[row];
     if (lane == 0) {
-      float* yp = y + (uint64_t)p * rows + row;
-      *yp = accumulate ? *yp + s : s;
+      const uint64_t yi = (uint64_t)p * rows + row;
+      y[yi] = add ? add[yi] + s : s;
     }
   }
 }
@@ -496,7 +496,7 @@ int spine_fast_launch(const SpineOp& op, int tail_lanes, int pg, int stream_wave
   const auto* w2 = static_cast<const uint8_t*>(op.w2);
   const auto* wb = static_cast<const uint8_t*>(op.wb);
   const int total_rows = op.rows + (op.wb ? op.rows_b : 0);
-  const int acc = op.accumulate ? 1 : 0;
+  const float* acc = op.add;
   TimedLaunch tl(KC_SPINE, st);
   bool launched_one = false;
   if (op.w2) {
@@ -613,8 +613,8 @@ int spine_gemv_op(int kind, const SpineOp& op, hipStream_t st) {
                       K3_SPINE_MAX_POSITIONS);
   if ((uint64_t)op.rows > (uint64_t)INT32_MAX / 2)
     return spine_fail(K3_SPINE_E_INVALID, "%s: too many rows", what);
-  if (op.w2 && op.accumulate)
-    return spine_fail(K3_SPINE_E_INVALID, "%s: a GLU projection does not accumulate", what);
+  if ((op.w2 || op.wb) && op.add)
+    return spine_fail(K3_SPINE_E_INVALID, "%s: only a single projection adds", what);
   if (op.wb && (op.w2 || !op.yb || op.rows_b <= 0 || (kind == K3_SPINE_KIND_INT8 && !op.scales_b) ||
                 (uint64_t)op.rows + op.rows_b > (uint64_t)INT32_MAX / 2))
     return spine_fail(K3_SPINE_E_INVALID, "%s: invalid second matrix", what);
@@ -632,7 +632,7 @@ int spine_gemv_op(int kind, const SpineOp& op, hipStream_t st) {
     sk.w2 = op.w2;
     sk.row_scales2 = op.scales2;
     sk.act = op.act;
-    sk.add = op.accumulate ? op.y : nullptr;
+    sk.add = op.add;
     sk.x = op.x;
     sk.x_dtype = K3_DTYPE_F32;
     sk.y = op.y;
@@ -690,10 +690,10 @@ int spine_gemv_op(int kind, const SpineOp& op, hipStream_t st) {
   TimedLaunch tl(KC_SPINE, st);
   if (kind == K3_SPINE_KIND_BF16)
     launch_timed(tl, k_spine_gemv_generic<K3_SPINE_KIND_BF16>, grid, dim3(kSpineThreads), 0, st,
-                 w, op.scales, op.x, op.y, op.rows, op.cols, op.positions, op.accumulate ? 1 : 0);
+                 w, op.scales, op.x, op.y, op.rows, op.cols, op.positions, op.add);
   else
     launch_timed(tl, k_spine_gemv_generic<K3_SPINE_KIND_INT8>, grid, dim3(kSpineThreads), 0, st,
-                 w, op.scales, op.x, op.y, op.rows, op.cols, op.positions, op.accumulate ? 1 : 0);
+                 w, op.scales, op.x, op.y, op.rows, op.cols, op.positions, op.add);
   const hipError_t e = hipGetLastError();
   if (e == hipSuccess) return K3_SPINE_OK;
   tl.failed();
@@ -701,7 +701,7 @@ int spine_gemv_op(int kind, const SpineOp& op, hipStream_t st) {
 }
 
 int spine_gemv(int kind, const void* weights, const float* row_scales, const float* x,
-               float* y, int rows, int cols, int positions, bool accumulate, hipStream_t st,
+               float* y, int rows, int cols, int positions, const float* add, hipStream_t st,
                bool any_order) {
   SpineOp op{};
   op.w = weights;
@@ -711,7 +711,7 @@ int spine_gemv(int kind, const void* weights, const float* row_scales, const flo
   op.rows = rows;
   op.cols = cols;
   op.positions = positions;
-  op.accumulate = accumulate;
+  op.add = add;
   op.any_order = any_order;
   return spine_gemv_op(kind, op, st);
 }
