@@ -39,8 +39,12 @@ __all__ = [
 
 
 def stream_handle(stream: torch.cuda.Stream | None = None) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return int(s.cuda_stream)
+    """The HIP stream of `stream`, or of the current device's current stream
+    (read as a handle: building a torch.cuda.Stream for it takes 2.8 us, a third
+    of a small call)."""
+    if stream is not None:
+        return int(stream.cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _dtype_code(t: torch.Tensor) -> int:

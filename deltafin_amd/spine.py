@@ -15,10 +15,7 @@ import ctypes as C
 import torch
 
 from . import _lib
-
-
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+from .moe import stream_handle
 
 
 def _dense(t: torch.Tensor, dtype: torch.dtype, what: str) -> None:
@@ -44,7 +41,7 @@ def bf16_gemv(weights: torch.Tensor, x: torch.Tensor, out: torch.Tensor | None =
     _dense(out, torch.float32, "out")
     lib = _lib.load()
     _lib.check_spine(lib.k3_hip_spine_bf16_launch_v1(
-        weights.data_ptr(), x2.data_ptr(), out.data_ptr(), rows, cols, x2.shape[0], _stream()),
+        weights.data_ptr(), x2.data_ptr(), out.data_ptr(), rows, cols, x2.shape[0], stream_handle()),
         "k3_hip_spine_bf16_launch_v1")
     return out
 
@@ -65,7 +62,7 @@ def int8_gemv(quantized: torch.Tensor, row_scales: torch.Tensor, x: torch.Tensor
     lib = _lib.load()
     _lib.check_spine(lib.k3_hip_spine_int8_launch_v1(
         quantized.data_ptr(), row_scales.data_ptr(), x2.data_ptr(), out.data_ptr(), rows, cols,
-        x2.shape[0], _stream()), "k3_hip_spine_int8_launch_v1")
+        x2.shape[0], stream_handle()), "k3_hip_spine_int8_launch_v1")
     return out
 
 
@@ -82,7 +79,7 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = _lib.K3_RMS_EPS
     _dense(out, torch.float32, "out")
     lib = _lib.load()
     _lib.check_spine(lib.k3_hip_rms_norm(x2.data_ptr(), weight.data_ptr(), out.data_ptr(),
-                                         x2.shape[0], x2.shape[1], float(eps), _stream()),
+                                         x2.shape[0], x2.shape[1], float(eps), stream_handle()),
                      "k3_hip_rms_norm")
     return out
 
@@ -95,7 +92,7 @@ def decode_bits(bits: torch.Tensor) -> torch.Tensor:
     out = torch.empty(bits.numel(), dtype=torch.int32, device=bits.device)
     lib = _lib.load()
     _lib.check_spine(lib.k3_hip_spine_bf16_decode_bits(bits.data_ptr(), out.data_ptr(),
-                                                       bits.numel(), _stream()),
+                                                       bits.numel(), stream_handle()),
                      "k3_hip_spine_bf16_decode_bits")
     return out
 
@@ -211,6 +208,6 @@ def moe_block(spine: MoeSpine, g, bank: torch.Tensor, stride: int, hidden: torch
     d = spine.descriptor()
     _lib.check(lib.k3_hip_moe_block_device(
         C.byref(d), C.byref(g), bank.data_ptr(), stride, h2.data_ptr(), P, out.data_ptr(),
-        ids.data_ptr(), wts.data_ptr(), workspace.data_ptr(), workspace.numel(), _stream()),
+        ids.data_ptr(), wts.data_ptr(), workspace.data_ptr(), workspace.numel(), stream_handle()),
         "k3_hip_moe_block_device")
     return out, ids, wts
