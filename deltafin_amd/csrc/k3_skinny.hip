@@ -5,12 +5,18 @@
 // one MXFP4 matrix against a batch of rows.
 //
 // Exactness.  An fp32 activation is split in registers into three BF16 terms
-// by truncation (the top 8 significant bits, the next 8, the last 8), so the
-// terms sum to it exactly; BF16, int8 and scaled E2M1 weights are exact in
-// BF16, and BF16 x BF16 products are exact in fp32, so only the summation
-// order differs from an fp32 FMA kernel.  Where a term product is not finite
-// although the fp32 sum may be (an infinite activation has a NaN remainder, an
-// infinite weight meets a zero term, a scaled code overflows BF16), the output
+// by truncation (the top 8 significant bits, the next 8, the last 8).  The two
+// lower terms are kept times 2^16 (kLowScale), which the sums' last step takes
+// back: unscaled they fall under BF16's smallest subnormal (2^-133) from
+// |x| < 2^-110 on, which lost 7e-5 of the result at 2^-120 (the multiply costs
+// 7168 x 6144 int8 at 16 positions 16.2 -> 16.7 us).  Scaled, the terms
+// sum to every finite fp32 value below 2^119 exactly, subnormals included (above,
+// the scaled remainder may overflow: see below).  BF16, int8 and scaled E2M1
+// weights are exact in BF16 and BF16 x BF16 products are exact in fp32 (the
+// matrix cores keep subnormal operands and sums), so only the summation order
+// differs from an fp32 FMA kernel.  Where a term product is not finite although
+// the fp32 sum may be (an infinite activation has a NaN remainder, an infinite
+// weight meets a zero term, a scaled code or remainder overflows), the output
 // comes out non-finite and the epilogue forms it again in plain fp32.
 //
 // Layout.  A wave reads whole 128-byte lines: one dwordx4 load covers 8 weight
@@ -47,6 +53,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint64_t u64_unaligned __attribute__((aligned(1)));
 
 constexpr int kMaxWaves = 8;
+constexpr float kLowScale = 65536.0f;  // of an fp32 activation's two lower terms
 
 // 32-column operands of a half line.
 template <int kW>
@@ -189,14 +196,15 @@ __device__ __forceinline__ void weight_operands(u32x4 w, uint32_t s, bf16x8 (&o)
   }
 }
 
-// Four fp32 values -> three truncated BF16 terms each.
+// Four fp32 values -> three truncated BF16 terms each, the second and third
+// times kLowScale.
 __device__ __forceinline__ void split4(u32x4 v, uint2 (&t)[3]) {
   uint32_t w[3][2];
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
     const uint32_t u0 = v[2 * e], u1 = v[2 * e + 1];
-    const float r0 = __uint_as_float(u0) - __uint_as_float(u0 & 0xffff0000u);
-    const float r1 = __uint_as_float(u1) - __uint_as_float(u1 & 0xffff0000u);
+    const float r0 = (__uint_as_float(u0) - __uint_as_float(u0 & 0xffff0000u)) * kLowScale;
+    const float r1 = (__uint_as_float(u1) - __uint_as_float(u1 & 0xffff0000u)) * kLowScale;
     const uint32_t m0 = __float_as_uint(r0), m1 = __float_as_uint(r1);
     const float l0 = r0 - __uint_as_float(m0 & 0xffff0000u);
     const float l1 = r1 - __uint_as_float(m1 & 0xffff0000u);
@@ -468,7 +476,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_skinny(const SkinnyArgs args
     for (int nb = 0; nb < NB; ++nb) {
       f32x4 v = acc[t][nb][0] + acc[t][nb][1];
 #pragma unroll
-      for (int c = 2; c < NA; ++c) v += acc[t][nb][c];
+      for (int c = 2; c < NA; ++c) v += NT > 1 ? acc[t][nb][c] * (1.0f / kLowScale) : acc[t][nb][c];
       sums[((wave * TLT + t) * NB + nb) * 64 + lane] = v;
     }
   __syncthreads();

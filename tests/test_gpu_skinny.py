@@ -124,6 +124,45 @@ def test_expert_rows(gpu, hidden, inter):
         _check(out, mats["down"], h.double(), inter, f"expert {hidden}/{inter} m{m}")
 
 
+# |x| around 1, where the lower terms of an fp32 activation are subnormal in BF16
+# (below 2^-110) and where x itself is subnormal
+EXPONENTS = [0, -100, -112, -120, -126, -132]
+
+
+@pytest.mark.parametrize("e", EXPONENTS)
+def test_small_activations(gpu, e):
+    """Activations of any size lose no bits: large weights bring every result to
+    about 1, and the results' distance from 64 bits in norm stays at fp32's.  A
+    sum is rounded once per matrix step or FMA, to 2^-24 of the partial sum; over
+    the 64 steps of 2,048 columns such errors add to about 8 x 2^-24 / sqrt(3) =
+    2.8e-7 of a sum of random signs.  4.8e-7 = 2^-21 is under twice that; a lost
+    third term costs 4e-6."""
+    import torch
+    from deltafin_amd import moe
+    rows, cols = 80, 2048
+    scale = 2.0 ** min(100, -e)
+
+    def near(y, ref, tag):
+        err = ((y.double() - ref).norm() / ref.norm()).item()
+        assert err <= 2.0 ** -21, f"{tag} at 2^{e}: {err:.2e}"
+
+    for m in (2, 7, 16):
+        print(f"[gpu-case] x at 2^{e}, {m} rows", flush=True)
+        x0 = torch.randn(m, cols, device="cuda", dtype=torch.float64)
+        x = (x0 * 2.0 ** e).float()
+        w, _, _, _ = _spine("bf16", rows, cols, m, m)
+        w = (w.float() * scale).to(torch.bfloat16)
+        near(_run_spine("bf16", w, None, x), x.double() @ w.double().t(), "bf16")
+        if e > -126:  # int8: the scale comes after the sum, which is subnormal below
+            w, s, _, w64 = _spine("int8", rows, cols, m, m)
+            near(_run_spine("int8", w, s * scale, x), x.double() @ (w64 * scale).t(), "int8")
+        p, _ = _mxfp4(rows, cols, m)
+        p &= 0xBB  # codes up to 1.5: exact in BF16 at every scale byte
+        s = torch.full((rows, cols // 32), 127 + int(min(100, -e)), device="cuda",
+                       dtype=torch.uint8)
+        near(moe.mxfp4_gemv(p, s, x, rows, cols), x.double() @ _dequant(p, s).t(), "mxfp4")
+
+
 def test_non_finite_inputs(gpu):
     """Infinities and NaN give what plain fp32 sums give: an infinite activation
     or weight its signed infinity, a NaN scale byte a NaN row, and a scale that
