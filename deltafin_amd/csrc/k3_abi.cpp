@@ -948,7 +948,7 @@ int from_spine(int rc, const char* step) {
 // decode layer per position on the device route.
 int experts_on_device_routes(const Geo& g, const uint8_t* bank, uint64_t stride, int n_bank,
                              int P, int top_k, const float* x, float* out, const Workspace& ws,
-                             hipStream_t st) {
+                             SideWork& side, hipStream_t st) {
   const int n_edges = P * top_k;
   const int mode = g_verify_mode.load();
   if (mode == K3_VERIFY_UNION_MFMA && !verify_mfma_supported(g))
@@ -960,6 +960,14 @@ int experts_on_device_routes(const Geo& g, const uint8_t* bank, uint64_t stride,
     int rc = launch_verify_plan_bank(g, bank, stride, n_bank, P, top_k, ws, st,
                                      mfma ? x : nullptr, K3_DTYPE_F32);
     if (rc != K3_HIP_OK) return rc;
+    // The matrix-core kernels fill the chip with two persistent workgroups of
+    // 73 KB LDS per CU.  Started while a side kernel still holds 40-48 KB of some
+    // CUs, their second workgroup there found no 73 KB in one piece until the first
+    // had ended: gate/up took 375 to 742 us from call to call.  So the side work
+    // ends first; it is as long as the router, routed_down and the plan, so the
+    // wait is short.  K3 block, BF16, us at 7 / 11 / 16 positions: 419 / 638 /
+    // 735 to 870 -> 421 / 576 / 736.
+    if (mfma && (rc = side.join()) != K3_HIP_OK) return rc;
     return mfma ? launch_verify_mfma(g, n_edges, P, x, K3_DTYPE_F32, out, K3_DTYPE_F32, ws, st,
                                      true)
                 : launch_verify_layer(g, n_edges, P, x, K3_DTYPE_F32, out, K3_DTYPE_F32, ws, st);
@@ -1037,7 +1045,8 @@ int k3_hip_moe_block_device(const K3HipMoeSpineV1* spine, const K3HipGeometryV1*
   // The shared expert needs only the hidden rows, so all of it runs on the side
   // stream where there is one, beside the router and the routed experts (the
   // two streams' kernels share the CUs and fill each other's ramps), and the
-  // caller's stream waits for its output only before routed_up, which adds it.
+  // caller's stream waits for its output only before routed_up, which adds it
+  // (before the experts' matrix-core kernels where the batch takes them).
   // The next call's fork is recorded after this call's routed_up, so the side
   // stream never overwrites an output that is still to be read.  Every return
   // after the fork joins first, so the caller's stream is never ahead of the
@@ -1117,7 +1126,7 @@ int k3_hip_moe_block_device(const K3HipMoeSpineV1* spine, const K3HipGeometryV1*
     return rc;
   // the routed experts
   if ((rc = experts_on_device_routes(g, bank, expert_stride, E, P, top_k, b.routed_in,
-                                     b.routed_out, ws, st)))
+                                     b.routed_out, ws, side, st)))
     return rc;
   if (!side.parallel() && (rc = shared_expert(st))) return rc;
   if ((rc = side.join())) return rc;  // the shared expert's output
