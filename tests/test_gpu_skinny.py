@@ -203,3 +203,64 @@ def test_non_finite_inputs(gpu):
         ref = x.double() @ w.t()
         keep = [i for i in range(40) if i != 3]
         assert ((y - ref)[:, keep].abs() <= 1e-4 * (x.double().abs() @ w[keep].abs().t())).all()
+
+
+@pytest.mark.parametrize("rows,m", [(33, 3), (40, 16), (4100, 16), (8200, 5), (4200, 33)])
+@pytest.mark.parametrize("kind", ["bf16", "int8", "mxfp4"])
+def test_non_finite_tiles(gpu, kind, rows, m):
+    """Sums formed again at every place of a tile: each position but the last has an
+    infinity, a NaN or a value whose scaled remainder overflows in some column; the
+    outputs are those of float64, and the last position's stay what they are alone."""
+    import torch
+    from deltafin_amd import moe
+    inf = float("inf")
+    cols = 1056
+    print(f"[gpu-case] non-finite {kind} {rows}x{cols} positions {m}", flush=True)
+    if kind == "mxfp4":
+        p, s = _mxfp4(rows, cols, rows + m)
+        w64 = _dequant(p, s)
+        x = torch.randn(m, cols, device="cuda")
+        run = lambda x: moe.mxfp4_gemv(p, s, x, rows, cols)
+    else:
+        w, s, x, w64 = _spine(kind, rows, cols, m, rows + m)
+        run = lambda x: _run_spine(kind, w, s, x)
+    clean = x.clone()
+    for i in range(m - 1):
+        c = (7 + 131 * i) % cols
+        x[i, c] = (inf, -inf, float("nan"), 2.0 ** 120 * (1.0 + 2.0 ** -7 - 2.0 ** -20))[i % 4]
+    y, ref = run(x), x.double() @ w64.t()
+    assert torch.equal(torch.isnan(y), torch.isnan(ref))
+    assert torch.equal(torch.isinf(y), torch.isinf(ref))
+    assert torch.equal(torch.sign(y[torch.isinf(y)]).double(), torch.sign(ref[torch.isinf(y)]))
+    fin = torch.isfinite(ref)
+    tol = 1e-5 * (torch.nan_to_num(x.double(), 0.0, 0.0, 0.0).abs() @ w64.abs().t())
+    assert ((y.double() - ref).abs() <= tol)[fin].all()
+    assert torch.equal(y[-1], run(clean)[-1])
+
+
+def test_non_finite_cost(gpu):
+    """A call whose every output is formed again stays within a small multiple of an
+    ordinary one (one thread per output: 70 times; a wave per four: about 8)."""
+    import torch
+    for kind in ("bf16", "int8"):
+        w, s, x, _ = _spine(kind, 7168, 6144, 16, 1)
+
+        def us(x):
+            for _ in range(3):
+                _run_spine(kind, w, s, x)
+            best = 1e9
+            for _ in range(5):
+                a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+                a.record()
+                for _ in range(4):
+                    _run_spine(kind, w, s, x)
+                b.record()
+                b.synchronize()
+                best = min(best, a.elapsed_time(b) * 250)
+            return best
+
+        ordinary = us(x)
+        x[:, 5000] = float("inf")
+        again = us(x)
+        print(f"[gpu-case] {kind}: {ordinary:.1f} us, formed again {again:.1f} us", flush=True)
+        assert again <= 30 * ordinary, f"{kind}: {ordinary:.1f} us -> {again:.1f} us"
