@@ -1077,7 +1077,7 @@ int k3_hip_moe_block_device(const K3HipMoeSpineV1* spine, const K3HipGeometryV1*
     glu.rows = S;
     glu.cols = H;
     glu.positions = P;
-    glu.any_order = skinny;
+    glu.matrix_cores = skinny;
     int r = spine_gemv_op(kind, glu, s);
     if (r == K3_SPINE_E_UNSUPPORTED) {
       if ((r = from_spine(spine_gemv(kind, sp.shared_gate, sp.shared_gate_scales, hidden, b.gate,

@@ -241,8 +241,7 @@ int spine_fail(int status, const char* fmt, ...);
 // add (nullable): y = W x + add, [positions, rows], one fp32 add per output.
 int spine_gemv(int kind, const void* weights, const float* row_scales, const float* x,
                float* y, int rows, int cols, int positions, const float* add,
-               hipStream_t stream,
-               bool any_order = false);
+               hipStream_t stream, bool matrix_cores = false);
 // One spine projection with the fused forms: w2 (GLU): y = act(W x, W2 x) per
 // row (no add); wb: a second matrix's rows after W's (see below);
 // norm_w: x is first RMS-normed per position,
@@ -266,10 +265,11 @@ struct SpineOp {
   const float* scales_b;
   float* yb;
   int rows_b;
-  // The summation order may depend on the number of positions: several
-  // positions take the matrix cores (k3_skinny.hip) where the shape allows.
-  // Unset, a (row, position) sums in one order whatever the batch.
-  bool any_order;
+  // On the matrix cores (k3_skinny.hip) where the shape and alignment allow,
+  // else on the fp32 kernels.  Each sums a (row, position) in one order whatever
+  // the number of positions, but not in the other's: a caller whose results must
+  // not depend on the batch sets this by the matrix alone.
+  bool matrix_cores;
 };
 int spine_gemv_op(int kind, const SpineOp& op, hipStream_t stream);
 int spine_decode_bits(const uint16_t* in, uint32_t* out, int count, hipStream_t stream);

@@ -1,8 +1,9 @@
 // Skinny products y[p, r] = sum_c W[r, c] x[p, c] on the BF16 matrix cores
 // (v_mfma_f32_16x16x32_bf16) for a few activation rows and a resident weight
 // matrix stored as BF16 bits, row-scaled int8 or MXFP4, in one launch with no
-// scratch memory: the spine projections at several positions, one expert or
-// one MXFP4 matrix against a batch of rows.
+// scratch memory: the spine projections, one expert or one MXFP4 matrix against a
+// batch of rows.  An output is summed in one order whatever the number of rows
+// beside it: the split and the order of a row's lines follow from its length.
 //
 // Exactness.  An fp32 activation is split in registers into three BF16 terms
 // by truncation (the top 8 significant bits, the next 8, the last 8).  The two

@@ -620,11 +620,7 @@ int spine_gemv_op(int kind, const SpineOp& op, hipStream_t st) {
     return spine_fail(K3_SPINE_E_INVALID, "%s: invalid second matrix", what);
   int rc = preflight(what);
   if (rc != K3_SPINE_OK) return rc;
-  // From two positions (three below 2,048 rows, where the launch is all ramp:
-  // 896 x 7168 at two 9.0 us against 7.8) the matrix cores read each weight
-  // once for all of them; 3584 x 7168 BF16, us at 2 / 4 / 16 / 64 positions:
-  // 14.7 / 22.6 / 68.7 / 241.9 -> 11.0 / 11.2 / 16.7 / 28.0.
-  if (op.any_order && !op.norm_w && !op.wb && op.positions >= (op.rows < 2048 ? 3 : 2)) {
+  if (op.matrix_cores && !op.norm_w && !op.wb) {
     SkinnyOp sk{};
     sk.kind = kind == K3_SPINE_KIND_BF16 ? SKINNY_BF16 : SKINNY_INT8;
     sk.w = op.w;
@@ -702,7 +698,7 @@ int spine_gemv_op(int kind, const SpineOp& op, hipStream_t st) {
 
 int spine_gemv(int kind, const void* weights, const float* row_scales, const float* x,
                float* y, int rows, int cols, int positions, const float* add, hipStream_t st,
-               bool any_order) {
+               bool matrix_cores) {
   SpineOp op{};
   op.w = weights;
   op.scales = row_scales;
@@ -712,7 +708,7 @@ int spine_gemv(int kind, const void* weights, const float* row_scales, const flo
   op.cols = cols;
   op.positions = positions;
   op.add = add;
-  op.any_order = any_order;
+  op.matrix_cores = matrix_cores;
   return spine_gemv_op(kind, op, st);
 }
 

@@ -11,6 +11,16 @@
 namespace k3 {
 namespace {
 thread_local char g_spine_error[512] = "no error";
+
+// The kernels of a public projection follow from the matrix alone, so that a
+// hidden row's result (a router's logits, say) has the same bits alone and in a
+// batch.  The matrix cores read the weights once for all positions; the fp32
+// kernels start faster, and few rows are all start.  BF16, us at 1 / 4 / 16 / 64
+// positions, fp32 against matrix cores: 640 x 7168 6.1 / 7.7 / 15.4 / 43 against
+// 9.0 / 9.4 / 15.0 / 13.8, 1536 x 7168 8.1 / 12.6 / 34 / 119 against 9.4 / 9.9 /
+// 15.6 / 18.8, 7168 x 6144 16.3 / 26 / 77 / 281 against 16.2 / 16.5 / 20.9 / 51.5
+// (int8 at one position: 5000 x 5120 8.1 against 9.7, 12288 x 7168 18 against 20).
+bool on_matrix_cores(int rows) { return rows >= 1024; }
 }  // namespace
 
 int spine_fail(int status, const char* fmt, ...) {
@@ -59,7 +69,7 @@ int k3_hip_spine_bf16_available(int device, int* compute_major, int* compute_min
 int k3_hip_spine_bf16_launch_v1(const uint16_t* weights, const float* activation, float* output,
                                 int rows, int columns, int positions, void* stream) {
   return spine_gemv(K3_SPINE_KIND_BF16, weights, nullptr, activation, output, rows, columns,
-                    positions, nullptr, static_cast<hipStream_t>(stream), true);
+                    positions, nullptr, static_cast<hipStream_t>(stream), on_matrix_cores(rows));
 }
 
 int k3_hip_spine_bf16_decode_bits(const uint16_t* input, uint32_t* output, int count,
@@ -71,7 +81,7 @@ int k3_hip_spine_int8_launch_v1(const int8_t* quantized, const float* row_scales
                                 const float* activation, float* output, int rows, int columns,
                                 int positions, void* stream) {
   return spine_gemv(K3_SPINE_KIND_INT8, quantized, row_scales, activation, output, rows, columns,
-                    positions, nullptr, static_cast<hipStream_t>(stream), true);
+                    positions, nullptr, static_cast<hipStream_t>(stream), on_matrix_cores(rows));
 }
 
 int k3_hip_rms_norm(const float* input, const float* weight, float* output, int rows, int columns,

@@ -26,7 +26,8 @@ def _dense(t: torch.Tensor, dtype: torch.dtype, what: str) -> None:
 def bf16_gemv(weights: torch.Tensor, x: torch.Tensor, out: torch.Tensor | None = None
               ) -> torch.Tensor:
     """out[p, r] = sum_c bf16(weights[r, c]) * x[p, c] in fp32.  weights: BF16
-    bits as int16/uint16/bfloat16 [rows, cols]; x: fp32 [positions, cols]."""
+    bits as int16/uint16/bfloat16 [rows, cols]; x: fp32 [positions, cols].  A
+    position's result has the same bits alone and in any batch."""
     if weights.dtype not in (torch.int16, torch.uint16, torch.bfloat16):
         raise ValueError("weights must hold BF16 bits (int16, uint16 or bfloat16)")
     if weights.device.type != "cuda" or not weights.is_contiguous() or weights.dim() != 2:
@@ -48,7 +49,8 @@ def bf16_gemv(weights: torch.Tensor, x: torch.Tensor, out: torch.Tensor | None =
 
 def int8_gemv(quantized: torch.Tensor, row_scales: torch.Tensor, x: torch.Tensor,
               out: torch.Tensor | None = None) -> torch.Tensor:
-    """out[p, r] = row_scales[r] * sum_c quantized[r, c] * x[p, c] in fp32."""
+    """out[p, r] = row_scales[r] * sum_c quantized[r, c] * x[p, c] in fp32.  A
+    position's result has the same bits alone and in any batch."""
     _dense(quantized, torch.int8, "quantized")
     _dense(row_scales, torch.float32, "row_scales")
     x2 = x if x.dim() == 2 else x.view(1, -1)

@@ -23,6 +23,14 @@
  *     k3_hip_spine_last_error() (thread-local).
  * Every matrix is row-major [rows, columns] and dense; activations are fp32
  * [positions, columns], outputs fp32 [positions, rows], positions 1..64.
+ *
+ * Batch invariance: an output of a projection has the same bits at every
+ * `positions` (for buffers of the same 16-byte alignment): its summation order
+ * follows from the matrix alone.  Matrices of 1,024 rows or more run on the
+ * BF16 matrix cores, which multiply an exact three-term BF16 split of each
+ * activation and sum in fp32; smaller ones, and shapes whose rows are not whole
+ * 16-byte pieces, on fp32 FMAs.  k3_hip_moe_block_device's projections choose by
+ * the batch instead (its router is invariant, see there).
  */
 #include <stdint.h>
 

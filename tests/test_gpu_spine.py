@@ -137,6 +137,31 @@ def test_int8_shapes(gpu, rows, cols):
         _close(out.cpu().numpy(), S.spine_int8_f64(q, s, x_np), f"int8 {rows}x{cols} p{positions}")
 
 
+@pytest.mark.parametrize("kind", ["bf16", "int8"])
+@pytest.mark.parametrize("rows,cols", [(896, 7168), (1023, 1040), (1024, 1040), (3584, 7168),
+                                       (8704, 2048), (1100, 8208), (2049, 1004), (12, 8208)])
+def test_positions_do_not_change_bits(gpu, kind, rows, cols):
+    """A hidden row's result is the same alone and at every place of a batch: on the
+    fp32 kernels (below 1,024 rows; 1,004 columns: the any-shape path), and on the
+    matrix cores at every tile and position-group size."""
+    import torch
+    from deltafin_amd import spine
+    gen = torch.Generator(device="cuda").manual_seed(rows + cols)
+    x = torch.randn(64, cols, generator=gen, device="cuda")
+    if kind == "bf16":
+        w = torch.randn(rows, cols, generator=gen, device="cuda").to(torch.bfloat16)
+        run = lambda x: spine.bf16_gemv(w, x)
+    else:
+        q = torch.randint(-128, 128, (rows, cols), generator=gen, device="cuda", dtype=torch.int8)
+        s = torch.rand(rows, generator=gen, device="cuda") + 0.5
+        run = lambda x: spine.int8_gemv(q, s, x)
+    alone = torch.cat([run(x[i:i + 1].clone()) for i in range(64)])
+    for positions in (2, 3, 4, 5, 8, 9, 16, 17, 33, 64):
+        say(f"{kind} {rows}x{cols} alone and among {positions}")
+        first = 64 - positions
+        assert torch.equal(run(x[first:].clone()), alone[first:]), f"{positions} positions"
+
+
 def test_decode_bits_exhaustive(gpu):
     import torch
     from deltafin_amd import spine
