@@ -2946,14 +2946,16 @@ int gemv1_dispatch(const uint8_t* p, const uint8_t* s, const XT* x, OT* y, int r
   return launched(tl, "mxfp4 GEMV launch");
 }
 
+// Activation bytes k_gemv_multi stages, so the widest row a call takes: also of
+// the calls that go to other kernels, so that the limit is the same at every
+// number of rows and every alignment.
+constexpr size_t kMultiLds = 64 * 1024;
+
 template <typename XT, typename OT>
 int gemv_multi_dispatch(const uint8_t* p, const uint8_t* s, const XT* x, OT* y, int rows,
                         int cols, int batches, hipStream_t st) {
   const size_t per = (size_t)cols * sizeof(XT);
-  const size_t budget = 64 * 1024;
-  int group = (int)std::min<size_t>(budget / per, (size_t)kMultiMax);
-  if (group < 1) return fail(K3_HIP_E_INVALID, "mxfp4 GEMV: cols=%d too wide for LDS staging", cols);
-  group = std::min(group, batches);
+  const int group = std::min((int)std::min<size_t>(kMultiLds / per, (size_t)kMultiMax), batches);
   const int waves = (rows + kRowsGemv - 1) / kRowsGemv;
   TimedLaunch tl(KC_GEMV, st);
   launch_timed(tl, (k_gemv_multi<XT, OT, kRowsGemv>), dim3((waves + 3) / 4), dim3(256),
@@ -2970,6 +2972,8 @@ int gemv_typed(const uint8_t* p, const uint8_t* s, const void* x, void* y, int r
     const int rc = gemv1_dispatch<XT, OT>(p, s, xt, yt, rows, cols, st);
     if (rc != -1) return rc;
   }
+  if ((size_t)cols * sizeof(XT) > kMultiLds)
+    return fail(K3_HIP_E_INVALID, "mxfp4 GEMV: cols=%d too wide", cols);
   // Several rows: on the matrix cores (3072 x 3584, fp32 x, us at 2 / 7 / 16
   // rows: 22.2 / 62.5 / 133.9 -> 5.8 / 7.0 / 8.5).
   SkinnyOp sk{};

@@ -96,6 +96,21 @@ def test_mxfp4_edges(gpu, cols, x_dtype):
                        out == torch.bfloat16)
 
 
+def test_mxfp4_widest_row(gpu):
+    """64 KB of activation is the widest row, whatever the number of rows."""
+    import torch
+    from deltafin_amd import _lib, moe
+    for dt, cols in ((torch.float32, 16384), (torch.bfloat16, 32768)):
+        for m in (1, 2, 5):
+            x = torch.randn(m, cols, device="cuda").to(dt)
+            p, s = _mxfp4(17, cols, m)
+            _check(moe.mxfp4_gemv(p, s, x, 17, cols), _dequant(p, s), x.double(), cols, f"{dt} m{m}")
+            p, s = _mxfp4(17, cols + 32, m)
+            x = torch.randn(m, cols + 32, device="cuda").to(dt)
+            with pytest.raises(_lib.K3HipError, match="too wide"):
+                moe.mxfp4_gemv(p, s, x, 17, cols + 32)
+
+
 @pytest.mark.parametrize("hidden,inter", [(256, 256), (3584, 3072), (1056, 352), (224, 64)])
 def test_expert_rows(gpu, hidden, inter):
     """moe_launch at 1..17 rows (224 / 64: below a whole line, the separate launches)."""
