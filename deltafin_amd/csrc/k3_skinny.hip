@@ -634,7 +634,8 @@ bool skinny_fits(const SkinnyOp& op) {
          row_bytes >= (op.kind == SKINNY_FP4 ? 128u : 64u) && op.cols <= 65536 &&
          op.positions <= (1 << 19) && (uint64_t)op.positions * op.cols <= (1u << 28) &&
          (uint64_t)op.positions * op.rows <= INT32_MAX && aligned16(op.w) && aligned16(op.x) &&
-         (!op.w2 || (aligned16(op.w2) && op.x_dtype == K3_DTYPE_F32));
+         (!op.w2 || (aligned16(op.w2) && op.x_dtype == K3_DTYPE_F32)) &&
+         !(op.add && (op.w2 || op.out_bf16));
 }
 
 int launch_skinny(const SkinnyOp& op, int kernel_class, hipStream_t st) {
