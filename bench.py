@@ -1090,18 +1090,16 @@ def _traffic_from_profiles(kernel: str):
 MFMA_PEAK_FP8_TFLOPS = 5000.0
 MFMA_FLOPS = 2 * 16 * 16 * 128  # one 16x16x128 block-scaled MFMA
 X_TERMS, H_TERMS = 2, 3         # fp8 terms per bf16 x row / fp32 h row
-PARITY_SPLIT = 2                # MFMA rows per weight row in a parity-split tile
 
 
 def _mfma_issued_per_expert() -> int:
     """MFMA instructions the union kernels issue per unique expert: gate and up
     (I/16 row tiles each, H/128 K steps, one per x term) and down (H/16 row
-    tiles, I/128 K steps, one per h term), times 2 for the parity split (a
-    tile's 16 MFMA rows hold 8 weight rows, each as an even and an odd K
-    step).  Each covers 16 token columns."""
+    tiles, I/128 K steps, one per h term).  Each covers 16 weight rows (two tiles
+    of 8, whose lanes exchange halves) and 16 token columns."""
     glu = 2 * (INTER // 16) * (HIDDEN // 128) * X_TERMS
     down = (HIDDEN // 16) * (INTER // 128) * H_TERMS
-    return PARITY_SPLIT * (glu + down)
+    return glu + down
 
 
 VERIFY_SETTLE_S = 0.05
@@ -1224,8 +1222,8 @@ def _verify_batches(moe, _lib, g, bank, stride, logits, x, batches: int) -> dict
         if kus.get("down_mfma") else None,
         # Useful = the layer's own multiply-adds (2 flops per weight and real
         # token) over the two matrix-core kernels' time; issued = every MFMA
-        # the kernels issue (16 token columns each, padding and parity split
-        # included), which is what keeps the matrix cores busy.
+        # the kernels issue (16 token columns each, padding included),
+        # which is what keeps the matrix cores busy.
         "mfma_util": round(useful / mfma_s / (MFMA_PEAK_FP8_TFLOPS * 1e12), 5) if mfma_s else None,
         "mfma_useful_tflops": round(useful / mfma_s / 1e12, 2) if mfma_s else None,
         "mfma_issued_tflops": round(issued / mfma_s / 1e12, 1) if mfma_s else None,
@@ -1602,8 +1600,7 @@ def _verify_config3(moe, _lib, g, bank, stride, batches: int,
                       "kernels (every routed expert read once per batch); mfma_util = the "
                       "layer's useful flops (2 per weight and routed token) / (gate/up + down "
                       "matrix-core kernel time x 5.0 PFLOP/s dense fp8); mfma_issued_util counts "
-                      "every issued block-scaled MFMA (16 token columns each, padding and the "
-                      "parity split included)",
+                      "every issued block-scaled MFMA (16 token columns each, padding included)",
             **out}
 
 

@@ -1,0 +1,11 @@
+"""bench.py's own figures and switches, without a GPU."""
+import bench
+
+
+def test_issued_matrix_products():
+    """One v_mfma_scale_f32_16x16x128 per 16 weight rows, K step of 128 and
+    activation term: the columns of all products together are the matrices'
+    elements times their terms."""
+    elements = {"glu": 2 * bench.INTER * bench.HIDDEN, "down": bench.HIDDEN * bench.INTER}
+    want = elements["glu"] * bench.X_TERMS + elements["down"] * bench.H_TERMS
+    assert bench._mfma_issued_per_expert() * 16 * 128 == want
