@@ -14,8 +14,8 @@ Printed: one JSON line with the step throughput, the roofline of the dominant
 kernel (algorithmic bytes per launch / average launch duration measured with
 HIP events on the launch stream), parity of sampled tokens against the fp64
 oracle, and the reference CPU path (tools/fused_gemv_batch.c, compiled from the
-reference sources into oracle/_ref) timed on this host over a bounded sample of
-the same tokens.
+reference sources into oracle/_ref, where they are present) timed on this host
+over a bounded sample of the same tokens.
 
     python bench.py [--steps K] [--warmup W] [--cpu-seconds S] [--no-cpu]
     python bench.py --copy-calibration   # plain 1 GiB device copies, for scaling
@@ -114,6 +114,18 @@ def parse() -> argparse.Namespace:
                     help="only run 4 plain device copies of 1 GiB (the known-size kernel "
                          "the HBM byte counters are scaled by) and exit")
     return ap.parse_args()
+
+
+def cpu_leg(asked: bool) -> bool:
+    """Whether the CPU baseline runs: asked for, and the reference's CPU library is
+    there (it is compiled from the reference's own sources, so only where they
+    are present).  Without it the line has no CPU figures (cpu_baseline null)."""
+    import oracle
+
+    if asked and not oracle.ref_available():
+        log(f"no CPU baseline: {oracle.REF_PATH.name} is not built")
+        return False
+    return asked
 
 
 COPY_CAL_BYTES = 1 << 30
@@ -556,6 +568,7 @@ def main() -> int:
     args = parse()
     if args.copy_calibration:
         return copy_calibration()
+    args.no_cpu = not cpu_leg(not args.no_cpu)
     if args.streamed:
         print(json.dumps(streamed_config4(args.streamed_tokens, not args.no_cpu)), flush=True)
         return 0

@@ -9,3 +9,12 @@ def test_issued_matrix_products():
     elements = {"glu": 2 * bench.INTER * bench.HIDDEN, "down": bench.HIDDEN * bench.INTER}
     want = elements["glu"] * bench.X_TERMS + elements["down"] * bench.H_TERMS
     assert bench._mfma_issued_per_expert() * 16 * 128 == want
+
+
+def test_cpu_leg_needs_its_library(monkeypatch):
+    """Without the reference's CPU library the line comes out with null baselines
+    instead of ending at the first of them."""
+    import oracle
+    for there, asked in ((True, True), (True, False), (False, True), (False, False)):
+        monkeypatch.setattr(oracle, "ref_available", lambda: there)
+        assert bench.cpu_leg(asked) == (there and asked)
