@@ -9,21 +9,21 @@ moe_block_f64):
   reference's bound max |out - expected| <= 2e-4 (:291);
 * the K3 geometry (hidden 7168, routed 3584, intermediate 3072, shared 6144,
   896 experts in a device bank) with BF16 spines at 1, 3, 4, 8, 11 and 16
-  positions (from 3 positions the spine runs on the BF16 matrix cores from
-  three-term activation splits; 11-16 take the three-tile form) and a
-  row-int8 spine at 2: every output within 1e-3 of the oracle relative to
+  positions and row-int8 spines at 2, 4 and 9 (from 3 positions every
+  projection but the router runs on the BF16 matrix cores from three-term
+  activation splits): every output within 1e-3 of the oracle relative to
   max(|ref|, mag / sqrt(n)) (oracle.cond_rel_err, mag = the size of the terms
   the output sums, n = routed + shared widths), route ids identical;
 * a small BF16 spine (hidden 576, routed 256, shared 320, 40 experts, top-8)
-  at 3 and 7 positions, where the matrix-core spine's row tails, single
-  column wave and zero-term padding run, under the same bar;
+  at 3 and 7 positions, where rows of 9, 4 and 5 lines split over as many
+  waves, under the same bar;
 * the route of a hidden row does not depend on the batch: the same rows at
   1, 4 and 16 positions route to the same experts with bit-identical weights;
 * 16 positions, where AUTO takes the union path: outputs equal the
   one-decode-layer-per-position path's within 1e-4 normwise, same routes;
 * calls at 1, 2 and 4 positions back to back on one workspace with no
-  synchronisation between them (the shared expert's gate/up runs on the
-  library's side stream and joins before shared_down): every call's output
+  synchronisation between them (the shared expert runs on the library's side
+  stream and joins before routed_up adds it): every call's output
   against the oracle (the other cases exercise the side stream at every
   position count);
 * two host threads, each on its own stream and workspace, issuing block calls
@@ -129,7 +129,8 @@ def _normwise(got, want):
 
 
 @pytest.mark.parametrize("kind,positions", [("bf16", 1), ("bf16", 3), ("bf16", 4), ("bf16", 8),
-                                            ("bf16", 11), ("bf16", 16), ("int8", 2)])
+                                            ("bf16", 11), ("bf16", 16), ("int8", 2),
+                                            ("int8", 4), ("int8", 9)])
 def test_block_k3_geometry(gpu, k3_bank, kind, positions):
     import torch
     from deltafin_amd import spine
@@ -156,9 +157,9 @@ SMALL = dict(hidden=576, routed=256, inter=128, shared=320, experts=40, top_k=8)
 
 @pytest.mark.parametrize("positions", [3, 7])
 def test_block_small_bf16_spine(gpu, positions):
-    """A BF16 spine whose shapes leave row tails (40 router rows), a single
-    column wave (256 columns) and zero-term padding steps on the matrix-core
-    spine, against the oracle per element."""
+    """A BF16 spine whose rows (576, 256 and 320 columns) are fewer lines than
+    a workgroup has waves, or split unevenly over them, against the oracle per
+    element."""
     import torch
     from deltafin_amd import _lib, moe, spine
     say(f"block: small BF16 spine (576/256/320, 40 experts), positions {positions}")
@@ -196,17 +197,17 @@ def test_block_small_bf16_spine(gpu, positions):
         assert err <= 1e-3, f"position {p}: cond rel err {err:.3e}"
 
 
-def test_block_routes_do_not_depend_on_batch(gpu, k3_bank):
-    """The same hidden rows in a 1-position call, a 4-position call (BF16
-    matrix-core spine) and a 16-position call route to the same experts with
-    bit-identical weights: the router logits are summed in one order at every
-    batch size."""
+@pytest.mark.parametrize("kind", ["bf16", "int8"])
+def test_block_routes_do_not_depend_on_batch(gpu, k3_bank, kind):
+    """The same hidden rows in a 1-position call, a 4-position call (matrix-core
+    spine) and a 16-position call route to the same experts with bit-identical
+    weights: the router logits are summed in one order at every batch size."""
     import torch
     from deltafin_amd import spine
     g, bank, stride, _ = k3_bank
-    say("block: routes at 1, 4 and 16 positions")
-    m = _k3_spine("bf16", 515)
-    sp = _spine_from("bf16", m)
+    say(f"block: routes at 1, 4 and 16 positions, {kind}")
+    m = _k3_spine(kind, 515)
+    sp = _spine_from(kind, m)
     rows = np.random.default_rng(515).standard_normal((16, K3["hidden"]), dtype=np.float32)
     ids1, w1 = [], []
     for p in range(4):
