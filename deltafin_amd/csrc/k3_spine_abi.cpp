@@ -12,15 +12,17 @@ namespace k3 {
 namespace {
 thread_local char g_spine_error[512] = "no error";
 
-// The kernels of a public projection follow from the matrix alone, so that a
-// hidden row's result (a router's logits, say) has the same bits alone and in a
-// batch.  The matrix cores read the weights once for all positions; the fp32
-// kernels start faster, and few rows are all start.  BF16, us at 1 / 4 / 16 / 64
-// positions, fp32 against matrix cores: 640 x 7168 6.1 / 7.7 / 15.4 / 43 against
-// 9.0 / 9.4 / 15.0 / 13.8, 1536 x 7168 8.1 / 12.6 / 34 / 119 against 9.4 / 9.9 /
-// 15.6 / 18.8, 7168 x 6144 16.3 / 26 / 77 / 281 against 16.2 / 16.5 / 20.9 / 51.5
-// (int8 at one position: 5000 x 5120 8.1 against 9.7, 12288 x 7168 18 against 20).
-bool on_matrix_cores(int rows) { return rows >= 1024; }
+// The public projections take the matrix cores at every number of positions, so
+// that a hidden row's result (a router's logits, say) has the same bits alone and
+// in a batch.  The fp32 kernels would start faster at one position and walk the
+// positions beyond: BF16, us at 1 / 4 / 16 / 64 positions, fp32 against matrix
+// cores, 896 x 7168 6.2 / 8.5 / 19.5 / 62 against 9.0 / 9.5 / 15.2 / 14.1,
+// 3584 x 7168 11.8 / 20 / 62 / 230 against 10.5 / 11.0 / 16.7 / 28.5, 7168 x 6144
+// 16.3 / 26 / 77 / 281 against 16.2 / 16.5 / 20.9 / 51.5; int8 at one position,
+// 2048 x 7168 6.6 against 8.8, 12288 x 7168 18 against 20, 7168 x 6144 11.4
+// against 11.2.  Their results lie further from 64 bits, too (1.2e-7 of the result
+// against 9e-8).
+constexpr bool kMatrixCores = true;
 }  // namespace
 
 int spine_fail(int status, const char* fmt, ...) {
@@ -69,7 +71,7 @@ int k3_hip_spine_bf16_available(int device, int* compute_major, int* compute_min
 int k3_hip_spine_bf16_launch_v1(const uint16_t* weights, const float* activation, float* output,
                                 int rows, int columns, int positions, void* stream) {
   return spine_gemv(K3_SPINE_KIND_BF16, weights, nullptr, activation, output, rows, columns,
-                    positions, nullptr, static_cast<hipStream_t>(stream), on_matrix_cores(rows));
+                    positions, nullptr, static_cast<hipStream_t>(stream), kMatrixCores);
 }
 
 int k3_hip_spine_bf16_decode_bits(const uint16_t* input, uint32_t* output, int count,
@@ -81,7 +83,7 @@ int k3_hip_spine_int8_launch_v1(const int8_t* quantized, const float* row_scales
                                 const float* activation, float* output, int rows, int columns,
                                 int positions, void* stream) {
   return spine_gemv(K3_SPINE_KIND_INT8, quantized, row_scales, activation, output, rows, columns,
-                    positions, nullptr, static_cast<hipStream_t>(stream), on_matrix_cores(rows));
+                    positions, nullptr, static_cast<hipStream_t>(stream), kMatrixCores);
 }
 
 int k3_hip_rms_norm(const float* input, const float* weight, float* output, int rows, int columns,

@@ -26,10 +26,10 @@
  *
  * Batch invariance: an output of a projection has the same bits at every
  * `positions` (for buffers of the same 16-byte alignment): its summation order
- * follows from the matrix alone.  Matrices of 1,024 rows or more run on the
- * BF16 matrix cores, which multiply an exact three-term BF16 split of each
- * activation and sum in fp32; smaller ones, and shapes whose rows are not whole
- * 16-byte pieces, on fp32 FMAs.  k3_hip_moe_block_device's projections choose by
+ * follows from the matrix alone.  Rows of at least 64 bytes and a multiple of 16
+ * run on the BF16 matrix cores, which multiply an exact three-term BF16 split of
+ * each activation and sum in fp32; other shapes, and buffers that are not 16-byte
+ * aligned, on fp32 FMAs.  k3_hip_moe_block_device's projections choose by
  * the batch instead (its router is invariant, see there).
  */
 #include <stdint.h>

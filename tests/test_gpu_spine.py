@@ -142,8 +142,8 @@ def test_int8_shapes(gpu, rows, cols):
                                        (8704, 2048), (1100, 8208), (2049, 1004), (12, 8208)])
 def test_positions_do_not_change_bits(gpu, kind, rows, cols):
     """A hidden row's result is the same alone and at every place of a batch: on the
-    fp32 kernels (below 1,024 rows; 1,004 columns: the any-shape path), and on the
-    matrix cores at every tile and position-group size."""
+    matrix cores at every tile and position-group size, and on the any-shape path
+    (1,004 columns)."""
     import torch
     from deltafin_amd import spine
     gen = torch.Generator(device="cuda").manual_seed(rows + cols)
