@@ -81,7 +81,7 @@ __global__ __launch_bounds__(256) void k_split_terms(const SrcT* __restrict__ sr
 // gate/up at 462 us against 416 (5.7 -> 6.3 TB/s) and down at 235 against 209.
 //
 // At a unit's last item every wave writes its tiles' partial sums to LDS
-// (two slots by unit parity, one barrier per unit) and wave w sums tile w
+// (slots by unit parity, one barrier per unit) and wave w sums tile w
 // (w + S, ...) over the waves in wave order, applies the activation (phase A)
 // and stores its tokens' rows.
 //
@@ -106,6 +106,13 @@ constexpr int kScaleLoads = 16;
 // bytes of two K steps and 8 scale bytes each.
 constexpr int kPackQuads = 4;
 constexpr int kPackBytes = 4 * kPackQuads * 256 + 64 * 8;  // every lane stores 8 bytes
+
+// Sum slots of a workgroup: two by unit parity, so that one barrier per unit is
+// enough; a wave alone needs no second one (its LDS operations run in order), and
+// without it eight one-wave workgroups fit a CU, with it seven (verify of 16
+// positions at hidden 1280, intermediate 768, fp32 x: 59.2 us with seven, 54.5
+// with eight).
+__host__ __device__ constexpr int sum_slots(int S) { return S > 1 ? 2 : 1; }
 
 template <int kTiles>
 struct MfmaA {  // weights: streamed from HBM, two items in flight
@@ -166,12 +173,13 @@ __global__ __launch_bounds__(256, 2) void k_verify_mfma(const Geo g, const Works
                                                         float* __restrict__ out) {
   constexpr int kM = kGlu ? 2 : 1;
   constexpr int kTiles = kM * NT;
-  // [2][S][kTiles][64] sums, then [S][64 * kScaleLoads] scales, then [S] packed rows
+  // [slots][S][kTiles][64] sums, then [S][64 * kScaleLoads] scales, then [S] packed rows
   extern __shared__ __attribute__((aligned(16))) float2 red[];
   __shared__ MfmaPlan pl;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int S = blockDim.x >> 6;
+  const int slots = sum_slots(S);
   const int r16 = lane & 15, qb = lane >> 4;
   const int prow = r16 >> 1, par = r16 & 1;  // weight row in the tile, K-step parity
   const int K = kGlu ? g.hidden : g.inter;
@@ -290,7 +298,7 @@ __global__ __launch_bounds__(256, 2) void k_verify_mfma(const Geo g, const Works
   float2 acc[kTiles];  // weight rows 2 qb and 2 qb + 1 of each tile, token r16
   auto epilogue = [&](int ui) {
     const int unit = b0 + ui * NWG;
-    const int slot_par = ui & 1;
+    const int slot_par = ui & (slots - 1);
     float2* mine = red + (size_t)(slot_par * S + wave) * kTiles * 64;
 #pragma unroll
     for (int t = 0; t < kTiles; ++t) mine[t * 64 + lane] = acc[t];
@@ -327,13 +335,13 @@ __global__ __launch_bounds__(256, 2) void k_verify_mfma(const Geo g, const Works
   };
 
   const uint32_t sh = 8u * qb;  // this lane group's byte in each scale dword
-  uint32_t* sblk_lds = reinterpret_cast<uint32_t*>(red + (size_t)2 * S * kTiles * 64) +
+  uint32_t* sblk_lds = reinterpret_cast<uint32_t*>(red + (size_t)slots * S * kTiles * 64) +
                        (size_t)wave * 64 * kScaleLoads;
   // This wave's packed term rows: [4 kPackQuads rows][16] pieces of 16 bytes (piece
   // c of row r at c ^ r % 16, which spreads the row-wise stores and the token-wise
   // reads over the banks), then the rows' scale bytes.
   u32x4* rows_lds = reinterpret_cast<u32x4*>(
-      reinterpret_cast<uint8_t*>(red) + (size_t)2 * S * kTiles * 64 * sizeof(float2) +
+      reinterpret_cast<uint8_t*>(red) + (size_t)slots * S * kTiles * 64 * sizeof(float2) +
       (size_t)S * 64 * kScaleLoads * sizeof(uint32_t) + (size_t)wave * kPackBytes);
   u32x2* rows_sc = reinterpret_cast<u32x2*>(rows_lds + 64 * kPackQuads);
 
@@ -589,12 +597,12 @@ int mfma_launch(const Geo& g, int n_edges, const Workspace& ws, const uint8_t* b
                           kGlu ? K3_MFMA_GLU_WAVES : K3_MFMA_DOWN_WAVES);
   if (S < 1) return fail(K3_HIP_E_INVALID, "verify: no column split fits this geometry");
   const int max_units = n_edges * (rows / (8 * NT));
-  const unsigned lds = (unsigned)(2 * S * kTiles * 64 * sizeof(float2) +
+  const unsigned lds = (unsigned)(sum_slots(S) * S * kTiles * 64 * sizeof(float2) +
                                   (size_t)S * 64 * kScaleLoads * sizeof(uint32_t) +
                                   (size_t)S * kPackBytes);
-  // eight resident waves per CU (two per SIMD, the kernel's register budget),
-  // or what a CU's 160 KB of LDS hold (one-wave workgroups)
-  const int per_cu = std::min(8 / S, (int)(160 * 1024 / (lds + sizeof(MfmaPlan))));
+  // eight resident waves per CU (two per SIMD, the kernel's register budget; the
+  // LDS of every split fits them)
+  const int per_cu = 8 / S;
   const int grid = std::max(1, std::min(per_cu * std::max(1, device_cu_count()), max_units));
   const void* kfn = reinterpret_cast<const void*>(k_verify_mfma<kGlu, NT, T>);
   if (!lds_fits(kfn, 64 * S, lds))
