@@ -869,7 +869,10 @@ int verify_table(const Geo& g, const EdgeTable& tbl, const void* x, int x_dtype,
 }
 
 // ---------------------------------------------------------------- MoE block
-// Positions from which the block's spine projections run on the matrix cores.
+// Positions from which the block's spine projections run on the matrix cores: at
+// 2 they are no faster than the fp32 kernels, which give two positions the bits of
+// one (K3 block, us on fp32 / matrix cores, BF16 188 / 187.5 at 2 positions, 275 /
+// 235 at 3; int8 172 / 171 and 264 / 217).
 constexpr int kBlockSkinnyPositions = 3;
 static_assert(sizeof(K3HipMoeSpineV1) == 144, "K3HipMoeSpineV1 layout changed");
 

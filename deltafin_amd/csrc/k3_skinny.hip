@@ -578,9 +578,15 @@ bool go(const SkinnyArgs& a, hipStream_t st, TimedLaunch& tl) {
   return true;
 }
 
-// Lines in flight per wave: two where the registers still hold two workgroups
-// per CU; MXFP4 lines bring four times the columns of BF16 ones, and there one
-// is as fast from two tiles up (7168 x 2048, 7 rows: 5.8 us against 6.7).
+// Lines in flight per wave: two, except for MXFP4 from two tiles up, whose lines
+// bring four times the columns of BF16 ones: there one is as fast or faster (7168
+// x 2048, 7 rows: 5.8 us against 6.7; one expert at 7 rows with one / two in its
+// gate/up: 3584 / 3072 16.4 / 16.5, 7168 / 2048 21.0 / 20.5, 7168 / 7168 37.4 /
+// 41.7).  Three, four and six lines of one BF16 or int8 tile measured the same or
+// slower than two (896 x 7168, 8 rows, BF16: 11.2 at two, 12.4 at four, 13.7 at
+// six), one line slower at few workgroups (3584 x 7168 BF16, 1 row: 14.4 against
+// 10.5).  Four tiles, and two of gate and two of up, need 158 to 231 registers:
+// one workgroup per CU.
 template <int kW, int TL>
 constexpr int depth() {
   return kW == SKINNY_FP4 && TL > 1 ? 1 : 2;
@@ -659,8 +665,9 @@ int launch_skinny(const SkinnyOp& op, int kernel_class, hipStream_t st) {
                                                                                   : op.cols / 2;
   a.lines = (row_bytes + 127) / 128;
   a.tail = row_bytes - 128 * (a.lines - 1);
-  // Eight waves split a row's lines (16 measured the same or slower, 4 slower
-  // at long rows).
+  // Eight waves split a row's lines (16 measured the same or slower, also at few
+  // rows: 896 x 7168 BF16 at 1 / 8 / 16 positions 9.2 / 12.7 / 16.3 us against 9.0 /
+  // 11.2 / 15.0; 4 slower at long rows).
   a.per = (a.lines + kMaxWaves - 1) / kMaxWaves;
   a.S = (a.lines + a.per - 1) / a.per;
   // The fewest tiles per workgroup that leave no more workgroups than CUs, up to

@@ -74,11 +74,14 @@ __global__ __launch_bounds__(256) void k_split_terms(const SrcT* __restrict__ sr
 // rows, K step ks + i % 2, block g, one dwordx4 load per tile and line (K steps
 // ks, ks + 1).  Neighbouring lanes of two tiles exchange halves (one DPP step), so
 // that one register holds K step ks of 16 rows and the other K step ks + 1: MFMA
-// row 2 i is row i of the first tile, 2 i + 1 row i of the second.  The unit's
-// scaled products are what bounds fp32 x and the down rows, with three terms:
-// multiplying each tile's two K steps in separate MFMA rows instead, which
-// needs no exchange and twice the MFMAs, ran the K3 block's 16-position
-// gate/up at 462 us against 416 (5.7 -> 6.3 TB/s) and down at 235 against 209.
+// row 2 i is row i of the first tile, 2 i + 1 row i of the second.  Multiplying
+// each tile's two K steps in separate MFMA rows instead, which needs no exchange
+// and twice the MFMAs, made the products the bound with three terms: the K3
+// block's 16-position gate/up took 462 us against 410 (5.7 -> 6.4 TB/s) and down
+// 235 against 206.  Now nothing but the weight stream is near it: throwaway builds
+// took, of 410 and 206 us, 390 and 202 without products, 392 and 203 without term
+// loads, 301 and 141 without weight loads (8 positions of 16 of 384, bf16 x: of
+// 256 and 140, 254 and 136, 252 and 140, 154 and 101).
 //
 // At a unit's last item every wave writes its tiles' partial sums to LDS
 // (slots by unit parity, one barrier per unit) and wave w sums tile w
@@ -173,6 +176,7 @@ __global__ __launch_bounds__(256, 2) void k_verify_mfma(const Geo g, const Works
                                                         float* __restrict__ out) {
   constexpr int kM = kGlu ? 2 : 1;
   constexpr int kTiles = kM * NT;
+  static_assert(kTiles % 4 == 0, "tiles go in pairs, pairs two at a time");
   // [slots][S][kTiles][64] sums, then [S][64 * kScaleLoads] scales, then [S] packed rows
   extern __shared__ __attribute__((aligned(16))) float2 red[];
   __shared__ MfmaPlan pl;
@@ -538,12 +542,12 @@ namespace {
 // 8-row tiles per unit: of gate and of up (4: 32 rows each, with bf16 x's
 // two terms and with fp32 x's three), and of down (8: 64 rows; the path
 // takes hidden sizes that are multiples of 128, so these units always fit).
-// Each keeps two items of weights and one of
-// activation terms within the 256 VGPRs of two waves per SIMD without
-// spilling (fp32 x at 4 tiles: 238, down at 8: 237).  More weight bytes per
-// item measured faster: fp32 x at 2 tiles (16 rows each) ran the K3 block's
-// 16-position gate/up at 607-634 µs against 465 µs at 4, and down at 7 tiles
-// the preset-2 16-position verify's down at 288-289 µs against 266 at 8.
+// Each keeps two items of weights and one of activation terms within the 256
+// VGPRs of two waves per SIMD without spilling.  More weight bytes per item
+// measured faster: fp32 x at 2 tiles (16 rows each) ran the K3 block's
+// 16-position gate/up at 497 us against 411 at 4, and down at 4 tiles 245 us
+// against 206 at 8 (preset 2, 16 positions: 312 against 264).  Tiles go in pairs
+// and pairs two at a time, so a unit of one matrix has 4 or 8.
 #ifndef K3_MFMA_GLU3_TILES
 #define K3_MFMA_GLU3_TILES 4
 #endif
