@@ -268,6 +268,21 @@ typedef __attribute__((address_space(1))) const u32x4 gu32x4;
 typedef __attribute__((address_space(1))) const uint8_t gu8;
 typedef __attribute__((address_space(1))) const uint32_t gu32;
 
+// Two loads of 8 weight rows x one 128-byte line each (lane parity: the line's
+// half) -> a[0] the first halves of all 16 rows, a[1] the second: neighbouring
+// lanes exchange halves, lane 2 i keeping row i of the first load, lane 2 i + 1
+// row i of the second.
+__device__ __forceinline__ void pair_halves(u32x4 (&a)[2], bool odd) {
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const uint32_t send = odd ? a[0][d] : a[1][d];
+    const uint32_t recv =
+        (uint32_t)__builtin_amdgcn_update_dpp(0, (int)send, 0xB1, 0xf, 0xf, false);  // lane ^ 1
+    a[0][d] = odd ? recv : a[0][d];
+    a[1][d] = odd ? a[1][d] : recv;
+  }
+}
+
 __device__ __forceinline__ u32x4 load_chunk(const uint8_t* p) {
   return __builtin_nontemporal_load((gu32x4*)(p));
 }

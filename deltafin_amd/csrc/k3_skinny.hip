@@ -111,23 +111,6 @@ struct Stage {
   uint64_t s[kW == SKINNY_FP4 ? TLT : 1];
 };
 
-__device__ __forceinline__ uint32_t dpp_xor1(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, false);
-}
-
-// a[0], a[1] (8 rows x one line each) -> half line 0 and half line 1 of 16 rows.
-__device__ __forceinline__ void pair_halves(u32x4 (&a)[2], bool odd) {
-#pragma unroll
-  for (int d = 0; d < 4; ++d) {
-    const uint32_t send = odd ? a[0][d] : a[1][d];
-    const uint32_t recv = dpp_xor1(send);
-    const uint32_t lo = odd ? recv : a[0][d];
-    const uint32_t hi = odd ? a[1][d] : recv;
-    a[0][d] = lo;
-    a[1][d] = hi;
-  }
-}
-
 __device__ __forceinline__ void swap16(uint32_t& a, uint32_t& b) {
   const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
   a = r[0];

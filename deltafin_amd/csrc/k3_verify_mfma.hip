@@ -150,23 +150,9 @@ __device__ __forceinline__ v8i b_operand(u32x4 lo, u32x4 hi) {
   return r;
 }
 
-// a[0], a[1] (8 rows x two K steps each, lane parity the K step) -> K step 0 and
-// K step 1 of 16 rows.
-__device__ __forceinline__ void pair_halves(u32x4 (&a)[2], bool odd) {
-#pragma unroll
-  for (int d = 0; d < 4; ++d) {
-    const uint32_t send = odd ? a[0][d] : a[1][d];
-    const uint32_t recv =
-        (uint32_t)__builtin_amdgcn_update_dpp(0, (int)send, 0xB1, 0xf, 0xf, false);  // lane ^ 1
-    a[0][d] = odd ? recv : a[0][d];
-    a[1][d] = odd ? a[1][d] : recv;
-  }
-}
-
 // Activation terms are re-read by every unit of their expert: ordinary
 // (cached) loads, unlike the streamed weight chunks.
 __device__ __forceinline__ u32x4 load_b16(const uint8_t* p) { return *(gu32x4*)(p); }
-
 
 template <bool kGlu, int NT, int T>
 __global__ __launch_bounds__(256, 2) void k_verify_mfma(const Geo g, const Workspace ws,
