@@ -1435,6 +1435,13 @@ SPINE_POSITIONS = (1, 4, 16)
 SPINE_ROTATE_BYTES = 600_000_000  # > the 256 MB Infinity Cache: every pass streams HBM
 
 
+def spine_launch_us(kern: dict) -> float:
+    """Microseconds per projection launch of a timing window, whichever kernel took
+    it: `spine_mfma` (matrix cores) or `spine_gemv` (fp32)."""
+    took = [kern[k] for k in ("spine_mfma", "spine_gemv") if k in kern]
+    return sum(v["total_ms"] for v in took) * 1e3 / sum(v["launches"] for v in took)
+
+
 def _spine_bench(launches: int = 24) -> dict:
     """Spine projections at the K3 shapes, BF16 and row-int8, at 1, 4 and 16
     positions: each shape is launched `launches` times over enough distinct
@@ -1482,7 +1489,7 @@ def _spine_bench(launches: int = 24) -> dict:
                     run(i)
                 torch.cuda.synchronize()
                 kern, _ = _lib.timing_end()
-                us = kern["spine_gemv"]["total_ms"] * 1e3 / kern["spine_gemv"]["launches"]
+                us = spine_launch_us(kern)
                 alg = mat_bytes + p * cols * 4 + p * rows * 4
                 res[f"p{p}"] = {"us": round(us, 2), "gbs": round(alg / us / 1e3, 1),
                                 "hbm_frac": round(alg / us / 1e3 / HBM_PEAK_GBS, 4)}

@@ -18,3 +18,10 @@ def test_cpu_leg_needs_its_library(monkeypatch):
     for there, asked in ((True, True), (True, False), (False, True), (False, False)):
         monkeypatch.setattr(oracle, "ref_available", lambda: there)
         assert bench.cpu_leg(asked) == (there and asked)
+
+
+def test_spine_launch_time_of_either_kernel():
+    gemv, mfma = {"total_ms": 0.24, "launches": 24}, {"total_ms": 0.36, "launches": 24}
+    assert abs(bench.spine_launch_us({"spine_gemv": gemv}) - 10.0) < 1e-9
+    assert abs(bench.spine_launch_us({"spine_mfma": mfma, "rms_norm": gemv}) - 15.0) < 1e-9
+    assert abs(bench.spine_launch_us({"spine_gemv": gemv, "spine_mfma": mfma}) - 12.5) < 1e-9
