@@ -186,6 +186,31 @@ def test_small_activations(gpu, e):
         near(moe.mxfp4_gemv(p, s, x, rows, cols), x.double() @ _dequant(p, s).t(), "mxfp4")
 
 
+def test_small_weights(gpu):
+    """Weights that are subnormal in BF16 (E8M0 bytes 1 to 3 with codes of 0.5, BF16
+    weights around 2^-130) count in full; byte 0 is +0."""
+    import torch
+    from deltafin_amd import moe
+    rows, cols = 40, 2048
+    for m in (2, 7, 16):
+        print(f"[gpu-case] small weights, {m} rows", flush=True)
+        x = torch.randn(m, cols, device="cuda") * 2.0 ** 100
+        w = (torch.randn(rows, cols, device="cuda", dtype=torch.float64) * 2.0 ** -130).to(
+            torch.bfloat16)
+        cases = [("bf16", _run_spine("bf16", w, None, x), x, w.double())]
+        p, _ = _mxfp4(rows, cols, m)
+        p &= 0x99  # codes 0 and 0.5
+        for byte in (0, 1, 2, 3):
+            s = torch.full((rows, cols // 32), byte, device="cuda", dtype=torch.uint8)
+            for v in (x, x.to(torch.bfloat16)):
+                cases.append((f"byte {byte} {v.dtype}", moe.mxfp4_gemv(p, s, v, rows, cols), v,
+                              _dequant(p, s)))
+        for tag, y, v, w64 in cases:
+            ref = v.double() @ w64.t()
+            err = (y.double() - ref).norm().item()
+            assert err <= 2.0 ** -21 * ref.norm().item(), f"{tag}, {m} rows: {err:.2e}"
+
+
 def test_non_finite_inputs(gpu):
     """Infinities and NaN give what plain fp32 sums give: an infinite activation
     or weight its signed infinity, a NaN scale byte a NaN row, and a scale that
